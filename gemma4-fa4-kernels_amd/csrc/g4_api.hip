@@ -8,6 +8,7 @@
 
 #include <algorithm>
 
+#include "g4_dkdv_split.h"
 #include "g4_kernels.h"
 
 namespace {
@@ -121,6 +122,16 @@ unsigned* sched_ptr(const g4_problem& p, void* ws) {
 int4* dq_list_ptr(const g4_problem& p, void* ws) {
   if (!g4::dq_list_bytes(p)) return nullptr;
   return (int4*)((char*)sched_ptr(p, ws) + g4::kSchedBytes);
+}
+size_t bwd_ws_bytes(const g4_problem& p) {
+  return fwd_ws_bytes(p) + g4::delta_bytes(p) + g4::ds_bytes(p) + g4::kSchedBytes +
+         g4::dq_list_bytes(p) + g4::acc_bytes(p);
+}
+// The split dK/dV launch's partial tiles, when the caller's workspace holds
+// them beyond the backward's own needs (g4_workspace_bytes phase 2).
+float* dkdv_split_ptr(const g4_problem& p, void* ws, size_t bytes) {
+  const size_t own = bwd_ws_bytes(p), part = g4::dkdv_split_bytes(p);
+  return part && bytes >= own + part ? (float*)((char*)ws + own) : nullptr;
 }
 float* acc_ptr(const g4_problem& p, void* ws) {
   if (!g4::acc_bytes(p)) return nullptr;
@@ -394,6 +405,79 @@ int split_chunks(const g4_problem& p, int* keys) {
   if (keys != nullptr) *keys = (int)(per * 32);
   return (int)n;
 }
+// Split dK/dV launch (g4_dkdv_split.h) against the launch by whole key tiles
+// (head dim 512: pairs of tiles) on the 256 CUs, in steps of the longest chain
+// of one CU (about 2.2 us at head dim 512, 1.9 us at 256).
+//  - Whole tiles of equal sequences: full rounds of the costliest item.  Of
+//    unequal packed sequences: the costliest item while every item has a CU,
+//    else the average plus part of the costliest item (measured: head dim 512,
+//    16 x 1000 tokens 1.26 x the average, [6000, 6000] 1.5 x; head dim 256,
+//    16 x 500 tokens 1.65 x).
+//  - Split: the average, each step 1.3 x as long (the parts walk different query
+//    rows at a time, so Q and dO come from beyond the L2: 2.7-2.9 us against
+//    2.2-2.4 at 4096-8192 tokens), plus set-up and the sum.
+// Measured, one causal sequence, head dim 512, whole / split us: 64 tokens
+// 51 / 59 (whole), 96: 93 / 56, 256: 194 / 64, 1000: 585 / 129, 2048: 1099 /
+// 392, 4096: 2140 / 1427, 5000: 2609 / 2157, 6000: 3123 / 3096 (whole), 8192:
+// 4872 / 5930 (whole), 9000: 10683 / 7241, 12000: 14238 / 13020.  Head dim 256:
+// 256 tokens 45 / 55 (whole), 512: 72 / 61, 777: 105 / 69, 1025: 133 / 81,
+// 1600: 144 / 127, 2048: 151 / 177 (whole), 2500: 287 / 202, 4096: 337 / 363
+// (whole).
+// Not for problems of more than four items per CU (the work queue balances
+// those), striped ones, head dim 512 with key metadata or a window (no adapter
+// makes such a call; not compiled), or more than 64 packed sequences.
+size_t dkdv_split_bytes(const g4_problem& p) {
+  const bool meta = (p.vision_ids != nullptr && p.bidirectional_vision) ||
+                    p.document_ids != nullptr;
+  if (p.head_dim == 512 && (meta || p.window > 0)) return 0;
+  const bool packed = p.cu_seqlens_q != nullptr;
+  if (packed && p.num_seqs > 64) return 0;
+  if (ds_stripes(p, nullptr, 0)) return 0;
+  const int bn = p.head_dim == 512 ? 64 : 128;
+  const int64_t nt = (p.seqlen_k + bn - 1) / bn;
+  const int64_t per_seq = p.head_dim == 512 ? (nt + 1) / 2 : nt;
+  const int64_t items = (int64_t)p.num_seqs * per_seq * p.num_kv_heads;
+  if (items > 4 * kSplitParts) return 0;
+  const int grp = p.num_q_heads / p.num_kv_heads;
+  SplitSeq q;  // a sequence of the largest lengths
+  q.init(p.seqlen_q, p.seqlen_k, bn, p.window, grp);
+  double longest = 0;  // item
+  for (int64_t r = 0; r < per_seq; ++r) {
+    double c = q.before((int)r + 1) - q.before((int)r);
+    if (p.head_dim == 512 && nt - 1 - r != r)
+      c += q.before((int)(nt - r)) - q.before((int)(nt - 1 - r));
+    longest = std::max(longest, c);
+  }
+  double total, whole;
+  const int64_t rest_k = p.total_k - p.seqlen_k;  // packed: keys of the other sequences
+  if (packed && p.num_seqs > 1 && rest_k < (int64_t)(p.num_seqs - 1) * p.seqlen_k) {
+    // the others' lengths are on the device: between as many as fit of the
+    // largest length and all equal
+    const double most = (double)p.total_k / p.seqlen_k * q.before((int)nt);
+    const int64_t rest_q = std::max<int64_t>(p.total_q - p.seqlen_q, 0);
+    SplitSeq o;
+    o.init((int)std::min(rest_q / (p.num_seqs - 1), rest_k / (p.num_seqs - 1)),
+           (int)(rest_k / (p.num_seqs - 1)), bn, p.window, grp);
+    total = p.num_kv_heads *
+            (most + q.before((int)nt) + (p.num_seqs - 1.0) * o.before(o.nt)) / 2;
+  } else {
+    total = (double)p.num_seqs * p.num_kv_heads * q.before((int)nt);
+  }
+  if (packed && p.num_seqs > 1) {
+    // items that exist: a pair of 64-key tiles or one 128-key tile
+    const double real = (double)p.total_k / 128 * p.num_kv_heads;
+    whole = real <= kSplitParts
+                ? longest
+                : (p.head_dim == 512 ? 1.0 : 1.4) * total / kSplitParts + 0.6 * longest;
+  } else {
+    whole = (double)((items + kSplitParts - 1) / kSplitParts) * longest;
+  }
+  const double parts = std::min<double>(kSplitParts, std::max(1.0, total / kSplitMinPart));
+  const double split = kSplitStep * total / parts + kSplitTileCost + kSplitSumSteps;
+  if (whole <= 1.05 * split) return 0;
+  return 2 * (size_t)kSplitParts * kSplitSlotFloats * 4 +
+         align256((kSplitParts + 1) * sizeof(SplitCut));
+}
 size_t split_bytes(const g4_problem& p) {
   const int n = split_chunks(p, nullptr);
   if (n == 0) return 0;
@@ -411,11 +495,9 @@ const char* g4_last_error(void) { return g_last_error.c_str(); }
 size_t g4_workspace_bytes(const g4_problem* p, int phase) {
   g_last_error.clear();
   if (check_problem(p) != G4_OK) return 0;
-  size_t b = fwd_ws_bytes(*p);
-  if (phase == 1)
-    b += g4::delta_bytes(*p) + g4::ds_bytes(*p) + g4::kSchedBytes + g4::dq_list_bytes(*p) +
-         g4::acc_bytes(*p);
-  return b;
+  if (phase == 1) return bwd_ws_bytes(*p);
+  if (phase == 2) return bwd_ws_bytes(*p) + g4::dkdv_split_bytes(*p);
+  return fwd_ws_bytes(*p);
 }
 
 int g4_attn_fwd(const g4_problem* p, const void* q, g4_layout ql, const void* k, g4_layout kl,
@@ -515,6 +597,7 @@ int g4_attn_bwd_dkdv(const g4_problem* p, const void* q, g4_layout ql, const voi
   a.dv = (__bf16*)dv;
   a.dkl = dkl;
   a.dvl = dvl;
+  a.split_part = dkdv_split_ptr(*p, ws, ws_bytes);
   hipError_t e = g4::launch_bwd_dkdv(a, (hipStream_t)stream);
   if (e != hipSuccess) return hip_fail(e, "backward dK/dV");
   return G4_OK;

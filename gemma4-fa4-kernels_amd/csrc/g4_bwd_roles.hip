@@ -43,6 +43,7 @@
 #include <atomic>
 #include <type_traits>
 
+#include "g4_dkdv_split.h"
 #include "g4_kernels.h"
 
 namespace g4 {
@@ -122,9 +123,31 @@ __device__ __forceinline__ bool ds_seq_skipped(const BwdParams& a, int64_t first
          (first_row < a.ds_row_lo || first_row >= (int64_t)a.ds_row_lo + a.ds_seq_rows);
 }
 
+// The steps of one tile that a part of the split launch runs, and where the
+// tile's partial goes (null: the tile is whole).
+struct SplitRun {
+  SplitCut from, to;
+  bool cut_lo, cut_hi;  // the run starts / ends inside the tile
+  float* part;
+};
+
+// A wave's 32 key x 256 accumulator as fp32 in register order: 1 KB per
+// store, read back in the same order by dkdv_split_sum_kernel.
+__device__ __forceinline__ void store_split_part(float* part, const f32x16 (&acc)[8], int wave,
+                                                 int lane) {
+  f32x4* dst = (f32x4*)part + wave * 2048 + lane;
+#pragma unroll
+  for (int b = 0; b < 8; ++b)
+#pragma unroll
+    for (int r4 = 0; r4 < 4; ++r4)
+      dst[(b * 4 + r4) * 64] = f32x4{acc[b][r4 * 4], acc[b][r4 * 4 + 1], acc[b][r4 * 4 + 2],
+                                     acc[b][r4 * 4 + 3]};
+}
+
 // ROT: the dh = 1 P waves read the Q tile rotated by 16 rows (see step_p).
 // STRIPED: one stripe of the striped stored-dS backward (BwdParams::ds_row_lo).
-template <bool META, bool ROT, bool STRIPED>
+// SPLIT: a run of a tile's steps, from it0 (g4_dkdv_split.h).
+template <bool META, bool ROT, bool STRIPED, bool SPLIT>
 struct RolesKernel {
   using C = RolesCfg;
   char G4_LDS* smem;
@@ -136,6 +159,8 @@ struct RolesKernel {
   int my_vid, my_doc;
   int grp, kvh, qt_lo, nqt;
   bool up;  // query tiles walked upward (else from the last one down)
+  int it0;      // SPLIT: the tile's first step of this run
+  float* part;  // SPLIT: where a cut tile's partial goes (null: a whole tile)
   int64_t tq;
   int64_t ds_row0;  // dS tile row of this sequence's first query tile
   uint32_t ds_lane;  // byte offset of this lane's dS run inside a tile
@@ -148,6 +173,7 @@ struct RolesKernel {
 
   __device__ __forceinline__ void coords(int it, int& qh, int& i0) const {
     const int sh = __builtin_ctz(grp);  // grp is 1, 2, 4 or 8
+    if constexpr (SPLIT) it += it0;
     qh = kvh * grp + (it & (grp - 1));
     i0 = (up ? qt_lo + (it >> sh) : qt_lo + nqt - 1 - (it >> sh)) * C::kBM;
   }
@@ -393,6 +419,8 @@ struct RolesKernel {
         step_ds(it & 1, it, nsteps);
     }
 
+    if constexpr (SPLIT)
+      if (part != nullptr) return store_split_part(part, acc, wave, lane);
     if (my_j >= sq.lk) return;
     __bf16* dst = PWAVE ? a->dv + tok_off(sq, s, sq.ktok, my_j, a->dvl) +
                               (int64_t)kvh * a->dvl.head_stride
@@ -427,13 +455,14 @@ struct RolesKernel {
 
 // One key tile kt of sequence s and KV head kvh; its query tiles are walked
 // upward with `up`, else from the last one down.
-template <bool META, bool QUEUE, bool STRIPED>
+template <bool META, bool QUEUE, bool STRIPED, bool SPLIT = false>
 __device__ __forceinline__ void dkdv_roles_tile(const BwdParams& a, char* smem_raw, int kvh,
-                                                int s, int kt, bool up) {
+                                                int s, int kt, bool up,
+                                                const SplitRun* run = nullptr) {
   // Rotation only in the one-item-per-workgroup launch: measured on config 2
   // (one 8192-token sequence) dK/dV 5.32 -> 5.17 ms, but 5.21 -> 5.89 ms in the
   // work-queue launch of config 4 (packed, 1-2048-token segments).
-  using K = RolesKernel<META, !QUEUE, STRIPED>;
+  using K = RolesKernel<META, !QUEUE, STRIPED, SPLIT>;
   using C = RolesCfg;
   K ker;
   ker.smem = (char G4_LDS*)smem_raw;
@@ -505,7 +534,13 @@ __device__ __forceinline__ void dkdv_roles_tile(const BwdParams& a, char* smem_r
     // (sequence stripes: rows from the stripe's first, ds_row_lo; else 0)
     ker.ds_row0 = ds_first_row(a, sq, ker.s) - a.ds_row_lo;
   }
-  const int nsteps = ker.nqt * ker.grp;
+  int nsteps = ker.nqt * ker.grp;
+  if constexpr (SPLIT) {
+    const int hi = run->cut_hi ? split_step(run->to, nsteps) : nsteps;
+    ker.it0 = run->cut_lo ? split_step(run->from, nsteps) : 0;
+    nsteps = hi - ker.it0;
+    ker.part = run->part;
+  }
   ker.ds_lane = (ker.kb * 32 + (ker.lane & 31)) * 64 + 32 * ker.dh + 8 * ker.h32;
   const int jc = min(ker.my_j, sq.lk - 1);
   ker.my_vid = ker.has_vid ? p.vision_ids[sq.ktok + jc] : -1;
@@ -656,7 +691,8 @@ struct Roles256Cfg {
   static_assert(kLdsBytes <= 160 * 1024, "LDS budget");
 };
 
-template <bool META>
+// SPLIT: as RolesKernel's.
+template <bool META, bool SPLIT>
 struct Roles256Kernel {
   using C = Roles256Cfg;
   char G4_LDS* smem;
@@ -667,6 +703,8 @@ struct Roles256Kernel {
   bool has_vid, has_doc, has_meta;
   int my_vid, my_doc;
   int grp, kvh, qt_lo, nqt;
+  int it0;
+  float* part;
   int64_t tq;
   int64_t ds_row0;  // dS tile row of this sequence's first query tile
   RowReader<C::kCPR> rrd;
@@ -677,6 +715,7 @@ struct Roles256Kernel {
 
   __device__ __forceinline__ void coords(int it, int& qh, int& i0) const {
     const int sh = __builtin_ctz(grp);
+    if constexpr (SPLIT) it += it0;
     qh = kvh * grp + (it & (grp - 1));
     i0 = (qt_lo + nqt - 1 - (it >> sh)) * C::kBM;
   }
@@ -839,6 +878,8 @@ struct Roles256Kernel {
       else
         step_ds(it & 1, it, nsteps);
     }
+    if constexpr (SPLIT)
+      if (part != nullptr) return store_split_part(part, acc, wave, lane);
     if (my_j >= sq.lk) return;
     __bf16* dst = PWAVE ? a->dv + tok_off(sq, s, sq.ktok, my_j, a->dvl) +
                               (int64_t)kvh * a->dvl.head_stride
@@ -856,12 +897,12 @@ struct Roles256Kernel {
   }
 };
 
-// Work item L: (KV head, sequence, key tile); with total > 0, only the key
-// tiles that exist (total of them per KV head; the SeqTiles table is in LDS).
-template <bool META, bool QUEUE>
-__device__ __forceinline__ void dkdv_roles256_item(const BwdParams& a, char* smem_raw, int L,
-                                                   int total = 0) {
-  using K = Roles256Kernel<META>;
+// Key tile kt of sequence s and KV head kvh.
+template <bool META, bool QUEUE, bool SPLIT = false>
+__device__ __forceinline__ void dkdv_roles256_tile(const BwdParams& a, char* smem_raw, int kvh,
+                                                   int s, int kt,
+                                                   const SplitRun* run = nullptr) {
+  using K = Roles256Kernel<META, SPLIT>;
   using C = Roles256Cfg;
   K ker;
   ker.smem = (char G4_LDS*)smem_raw;
@@ -875,19 +916,8 @@ __device__ __forceinline__ void dkdv_roles256_item(const BwdParams& a, char* sme
   ker.h32 = ker.lane >> 5;
 
   ker.grp = p.num_q_heads / p.num_kv_heads;
-  int kt;
-  if (total > 0) {
-    ker.kvh = L / total;
-    int local, nt;
-    SeqTiles::find_lds((const int G4_LDS*)(smem_raw + C::kLdsSeq), L % total, ker.s, local, nt);
-    kt = zigzag(local, nt);
-  } else {
-    const int per_kvh = a.num_seqs * a.ntiles;
-    ker.kvh = L / per_kvh;
-    const int rank = L % per_kvh;
-    ker.s = rank / a.ntiles;
-    kt = zigzag(rank % a.ntiles, a.ntiles);
-  }
+  ker.kvh = kvh;
+  ker.s = s;
   ker.sq = resolve_seq(p, ker.s);
   const Seq& sq = ker.sq;
   ker.j0 = kt * C::kBN;
@@ -927,7 +957,13 @@ __device__ __forceinline__ void dkdv_roles256_item(const BwdParams& a, char* sme
     ker.has_doc = false;
     ker.has_meta = ker.has_vid;
   }
-  const int nsteps = ker.nqt * ker.grp;
+  int nsteps = ker.nqt * ker.grp;
+  if constexpr (SPLIT) {
+    const int hi = run->cut_hi ? split_step(run->to, nsteps) : nsteps;
+    ker.it0 = run->cut_lo ? split_step(run->from, nsteps) : 0;
+    nsteps = hi - ker.it0;
+    ker.part = run->part;
+  }
   ker.ds_row0 = sq.packed ? sq.qtok / 32 + ker.s : (int64_t)ker.s * ((p.seqlen_q + 31) / 32);
   const int jc = min(ker.my_j, sq.lk - 1);
   ker.my_vid = ker.has_vid ? p.vision_ids[sq.ktok + jc] : -1;
@@ -948,6 +984,28 @@ __device__ __forceinline__ void dkdv_roles256_item(const BwdParams& a, char* sme
     ker.template run<true>(nsteps);
   else
     ker.template run<false>(nsteps);
+}
+
+// Work item L: (KV head, sequence, key tile); with total > 0, only the key
+// tiles that exist (total of them per KV head; the SeqTiles table is in LDS).
+template <bool META, bool QUEUE>
+__device__ __forceinline__ void dkdv_roles256_item(const BwdParams& a, char* smem_raw, int L,
+                                                   int total = 0) {
+  using C = Roles256Cfg;
+  int kvh, s, kt;
+  if (total > 0) {
+    kvh = L / total;
+    int local, nt;
+    SeqTiles::find_lds((const int G4_LDS*)(smem_raw + C::kLdsSeq), L % total, s, local, nt);
+    kt = zigzag(local, nt);
+  } else {
+    const int per_kvh = a.num_seqs * a.ntiles;
+    kvh = L / per_kvh;
+    const int rank = L % per_kvh;
+    s = rank / a.ntiles;
+    kt = zigzag(rank % a.ntiles, a.ntiles);
+  }
+  dkdv_roles256_tile<META, QUEUE>(a, smem_raw, kvh, s, kt);
 }
 
 // Persistent: a few workgroups per CU take (KV head, sequence, key tile)
@@ -976,6 +1034,109 @@ __global__ void __launch_bounds__(Roles256Cfg::kNT, 1) dkdv_roles256_kernel(BwdP
     }
   } else {
     dkdv_roles256_item<META, false>(a, smem_raw, xcd_remap(blockIdx.x, gridDim.x));
+  }
+}
+
+// ===========================================================================
+// Split dK/dV launch (g4_dkdv_split.h): workgroup g runs part g of the steps,
+// then dkdv_split_sum_kernel adds the partial tiles.
+// ===========================================================================
+
+template <int D, bool META>
+__global__ void __launch_bounds__(512, 1) dkdv_split_kernel(BwdParams a) {
+  using C = std::conditional_t<D == 512, RolesCfg, Roles256Cfg>;
+  static_assert(C::kNT == 512 && C::kNB == 8, "partial slot layout");
+  extern __shared__ __attribute__((aligned(16))) char smem_raw[];
+  const int g = xcd_remap(blockIdx.x, gridDim.x);
+  static_assert(sizeof(SplitScratch) <= C::kLdsLd, "the cuts' scratch lies in the tile area");
+  SplitCut* const cuts = (SplitCut*)(a.split_part + 2 * (size_t)kSplitParts * kSplitSlotFloats);
+  SplitRun run;
+  split_cuts<C::kNT>(a, C::kBN, g, (SplitScratch G4_LDS*)smem_raw, run.from, run.to);
+  // the cuts for dkdv_split_sum_kernel
+  if (threadIdx.x == 0) cuts[g] = run.from;
+  if (threadIdx.x == 1 && g == kSplitParts - 1) cuts[kSplitParts] = run.to;
+  if (g >= run.from.parts) return;
+  int kvh = run.from.kvh, s = run.from.s, kt = run.from.kt;
+  const int last = run.to.num > 0 ? run.to.unit : run.to.unit - 1;
+#pragma nounroll
+  for (int u = run.from.unit; u <= last; ++u) {
+    barrier_lds();  // every wave is done with the scratch, or the previous tile's LDS
+    run.cut_lo = u == run.from.unit && run.from.num > 0;
+    run.cut_hi = u == run.to.unit;
+    // slot 0: the tile was begun by an earlier part; slot 1: it begins here
+    run.part = run.cut_lo || run.cut_hi
+                   ? a.split_part + (2 * (size_t)g + (run.cut_lo ? 0 : 1)) * kSplitSlotFloats
+                   : nullptr;
+    if constexpr (D == 512)
+      dkdv_roles_tile<META, false, false, true>(a, smem_raw, kvh, s, kt, false, &run);
+    else
+      dkdv_roles256_tile<META, true, true>(a, smem_raw, kvh, s, kt, &run);
+    // the next key tile: of the sequence, of the next one that has keys, or of
+    // the next KV head's first one
+    ++kt;
+    while (u < last && kt * C::kBN >= resolve_seq(a.p, s).lk) {
+      kt = 0;
+      if (++s == a.num_seqs) {
+        s = 0;
+        ++kvh;
+      }
+    }
+  }
+}
+
+// Block (g - 1) * 8 + w adds wave w's accumulator (32 keys x 256 columns of dV
+// or dK) over the parts of the tile cut at the beginning of part g, when that
+// is the tile's first cut: part g - 1's start of the tile, then the parts
+// that go on with it in order.
+template <int D>
+__global__ void __launch_bounds__(256) dkdv_split_sum_kernel(BwdParams a) {
+  using C = std::conditional_t<D == 512, RolesCfg, Roles256Cfg>;
+  constexpr int kPitch = 512 + 16;  // bytes per staged row
+  __shared__ __attribute__((aligned(16))) char stage[32 * kPitch];
+  const int g = 1 + blockIdx.x / 8, w = blockIdx.x % 8;
+  const SplitCut* cuts =
+      (const SplitCut*)(a.split_part + 2 * (size_t)kSplitParts * kSplitSlotFloats);
+  const SplitCut cut = cuts[g];
+  if (g >= cut.parts || cut.num == 0) return;
+  if (cuts[g - 1].unit == cut.unit && cuts[g - 1].num > 0) return;  // an earlier cut's block
+  const f32x4* src = (const f32x4*)a.split_part + w * 2048 + threadIdx.x;
+  constexpr size_t kSlot4 = kSplitSlotFloats / 4;
+  f32x4 sum[8];
+#pragma unroll
+  for (int i = 0; i < 8; ++i) sum[i] = src[(2 * (size_t)(g - 1) + 1) * kSlot4 + i * 256];
+  for (int c = g;; ++c) {
+    f32x4 x[8];
+#pragma unroll
+    for (int i = 0; i < 8; ++i) x[i] = src[2 * (size_t)c * kSlot4 + i * 256];
+    const bool done = cuts[c + 1].unit != cut.unit || cuts[c + 1].num == 0;
+#pragma unroll
+    for (int i = 0; i < 8; ++i) sum[i] += x[i];
+    if (done) break;
+  }
+  // register order -> rows: element (b, r4) of lane l is key l & 31, columns
+  // 32 b + 8 r4 + 4 (l >> 5) ..
+#pragma unroll
+  for (int i = 0; i < 8; ++i) {
+    const int x = i * 256 + threadIdx.x;
+    const int lane = x & 63, r4 = (x >> 6) & 3, b = x >> 8;
+    *(bf16x4*)(stage + (lane & 31) * kPitch + (b * 32 + 8 * r4 + 4 * (lane >> 5)) * 2) =
+        bf16x4{(__bf16)sum[i][0], (__bf16)sum[i][1], (__bf16)sum[i][2], (__bf16)sum[i][3]};
+  }
+  __syncthreads();
+  const int kvh = cut.kvh, s = cut.s, kt = cut.kt;
+  const Seq sq = resolve_seq(a.p, s);
+  const int kb = D == 512 ? (w & 3) >> 1 : w & 3;
+  const int col = D == 512 ? 256 * (w & 1) : 0;
+  const int row = threadIdx.x >> 3;
+  const int j = kt * C::kBN + kb * 32 + row;
+  if (j >= sq.lk) return;
+  const g4_layout& ly = w < 4 ? a.dvl : a.dkl;
+  __bf16* dst = (w < 4 ? a.dv : a.dk) + tok_off(sq, s, sq.ktok, j, ly) +
+                (int64_t)kvh * ly.head_stride + col;
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    const int c = (threadIdx.x & 7) + 8 * i;
+    *(bf16x8*)(dst + c * 8) = *(const bf16x8*)(stage + row * kPitch + c * 16);
   }
 }
 
@@ -2054,10 +2215,25 @@ hipError_t launch_bwd_dq(const BwdParams& a, hipStream_t stream) {
 }
 
 template <int D>
+static hipError_t launch_dkdv_split(const BwdParams& a, bool meta, hipStream_t stream) {
+  using C = std::conditional_t<D == 512, RolesCfg, Roles256Cfg>;
+  void (*kern)(BwdParams) = meta ? dkdv_split_kernel<D, D == 256> : dkdv_split_kernel<D, false>;
+  static LdsAttr attr[2];
+  hipError_t e = attr[meta].ensure((const void*)kern, C::kLdsBytes);
+  if (e != hipSuccess) return e;
+  hipLaunchKernelGGL(kern, dim3(kSplitParts), dim3(C::kNT), C::kLdsBytes, stream, a);
+  e = hipGetLastError();
+  if (e != hipSuccess) return e;
+  hipLaunchKernelGGL(dkdv_split_sum_kernel<D>, dim3((kSplitParts - 1) * 8), dim3(256), 0, stream, a);
+  return hipGetLastError();
+}
+
+template <int D>
 hipError_t launch_dkdv_roles_d(const BwdParams& a, hipStream_t stream) {
   using C = std::conditional_t<D == 512, RolesCfg, Roles256Cfg>;
   const bool meta = (a.p.vision_ids != nullptr && a.p.bidirectional_vision) ||
                     a.p.document_ids != nullptr;
+  if (a.split_part != nullptr) return launch_dkdv_split<D>(a, meta, stream);
   BwdParams b = a;
   b.ntiles = (a.p.seqlen_k + C::kBN - 1) / C::kBN;
   // Head dim 512: one item per pair of key tiles (see dkdv_roles_pair).

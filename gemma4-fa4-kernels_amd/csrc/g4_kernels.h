@@ -98,6 +98,9 @@ struct BwdParams {
   // Head dim 256 dQ after the stored-dS pass: only the query tiles whose vision
   // spans reach past the stored band (set by the launcher).
   int dq_recompute_only;
+  // Split dK/dV launch (g4_dkdv_split.h): the parts' fp32 partial tiles, two
+  // slots of kSplitSlotFloats per part, or null for the launch by whole tiles.
+  float* split_part;
   // Work-queue ticket counters of the persistent tile kernels: [0] dK/dV,
   // [2] dQ; zeroed by the delta pass, and by each launch's last draw.  [3]
   // counts the entries of dq_list.
@@ -199,6 +202,12 @@ size_t acc_bytes(const g4_problem& p);
 int split_chunks(const g4_problem& p, int* keys);
 // Workspace bytes of its partial rows (0 when not split).
 size_t split_bytes(const g4_problem& p);
+// Split dK/dV launch: parts (one per CU of the MI355X), floats of one partial
+// slot (the dK and dV of one key tile, 64 x 512 or 128 x 256 each), and the
+// workspace bytes of the slots: 0 when the launch by whole tiles is as good.
+constexpr int kSplitParts = 256;
+constexpr size_t kSplitSlotFloats = 2 * 64 * 512;
+size_t dkdv_split_bytes(const g4_problem& p);
 int64_t k_stream_tokens(const g4_problem& p);
 int64_t q_stream_tokens(const g4_problem& p);
 

@@ -535,6 +535,10 @@ class _Plan:
     # Global layers fail closed at backward time when even the recompute route
     # does not fit the guarded budget (GlobalBackwardBudgetExceeded).
     global_backward: bool = False
+    # Additional bytes that fit at backward time beyond what the chosen route
+    # needs (0 with a pinned dS budget): the split dK/dV launch's partial tiles
+    # are taken from them (g4_workspace_bytes phase 2).
+    spare_bytes: int = 0
     # Cumulative-array checks still to run before the first launch.
     pending: _CumulativeCheck | None = field(default=None, repr=False, compare=False)
     # Workspace sizes already asked of the library, by (phase, ds_budget): the
@@ -592,6 +596,10 @@ class _Plan:
 
     def _workspace(self, phase: int, device, prob: G4Problem | None = None) -> torch.Tensor:
         nbytes = max(self.workspace_bytes(phase, prob), 256)
+        if phase == 1 and self.spare_bytes > 0:
+            split = self.workspace_bytes(2, prob)
+            if split - nbytes <= self.spare_bytes:
+                nbytes = max(nbytes, split)
         return torch.empty(nbytes, dtype=torch.uint8, device=device)
 
     def forward(self, q, k, v):
@@ -876,6 +884,8 @@ def _refit_backward(plan: _Plan, q, k, v) -> None:
     """
     free = _free_hbm(q.device)
     required = _fit_or_pin(plan, q, k, v, free)
+    plan.spare_bytes = 0 if _PINNED_DS_BUDGET is not None else \
+        _global_backward_budget(free) - required
     if plan.global_backward:
         _check_global_backward_budget(required, free)
 

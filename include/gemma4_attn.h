@@ -92,7 +92,12 @@ const char* g4_last_error(void);
 
 /* Bytes of workspace g4_attn_fwd (phase 0) or g4_attn_bwd (phase 1) needs.
  * Returns 0 and sets the error on an invalid problem.  A valid problem that
- * needs no workspace (0 bytes) may pass a NULL workspace. */
+ * needs no workspace (0 bytes) may pass a NULL workspace.
+ * Phase 2: phase 1 plus, for a problem whose key tiles do not fill the GPU
+ * evenly, 128 MiB for fp32 partial dK / dV tiles.  A backward given at least
+ * that much cuts its dK / dV work into equal parts over the CUs and adds the
+ * partials in a fixed order; dQ is bitwise the same, dK / dV differ by the
+ * order of the fp32 sums.  Equal to phase 1 when the split would not pay. */
 size_t g4_workspace_bytes(const g4_problem* p, int phase);
 
 /*
