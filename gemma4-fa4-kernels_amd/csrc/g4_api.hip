@@ -177,7 +177,7 @@ int scratch_for_stream(hipStream_t stream, void** out) {
 
 int fwd_impl(const g4_problem* p, const void* q, g4_layout ql, const void* k, g4_layout kl,
              const void* v, g4_layout vl, void* o, g4_layout ol, float* lse, void* ws,
-             hipStream_t st) {
+             size_t ws_bytes, hipStream_t st) {
   g4::FwdParams a{};
   a.p = *p;
   a.q = (const __bf16*)q;
@@ -197,7 +197,10 @@ int fwd_impl(const g4_problem* p, const void* q, g4_layout ql, const void* k, g4
   g4::span_arrays(*p, ws, &a.span_lo, &a.span_hi);
   a.raise_flags = raise_flags_ptr(*p, ws);
   a.part = split_ptr(*p, ws);
-  if (a.part != nullptr) a.split_chunks = g4::split_chunks(*p, &a.split_keys);
+  if (a.part != nullptr)
+    a.split_chunks = g4::split_chunks(*p, &a.split_keys);
+  else if (const size_t wide = g4::wide_split_bytes(*p); wide && ws_bytes >= fwd_ws_bytes(*p) + wide)
+    a.part = (float*)((char*)ws + fwd_ws_bytes(*p));
   if (unsigned* dl = fwd_doc_list_ptr(*p, ws)) {
     a.doc_list_n = dl;
     a.doc_list = (int*)(dl + 64);
@@ -497,6 +500,8 @@ size_t g4_workspace_bytes(const g4_problem* p, int phase) {
   if (check_problem(p) != G4_OK) return 0;
   if (phase == 1) return bwd_ws_bytes(*p);
   if (phase == 2) return bwd_ws_bytes(*p) + g4::dkdv_split_bytes(*p);
+  if (phase == 3)
+    return fwd_ws_bytes(*p) + (g4::split_bytes(*p) ? 0 : g4::wide_split_bytes(*p));
   return fwd_ws_bytes(*p);
 }
 
@@ -506,7 +511,7 @@ int g4_attn_fwd(const g4_problem* p, const void* q, g4_layout ql, const void* k,
   g_last_error.clear();
   G4_TRY(check_fwd_operands(p, q, ql, k, kl, v, vl, o, ol, lse));
   G4_TRY(check_ws(p, 0, ws, ws_bytes));
-  return fwd_impl(p, q, ql, k, kl, v, vl, o, ol, lse, ws, (hipStream_t)stream);
+  return fwd_impl(p, q, ql, k, kl, v, vl, o, ol, lse, ws, ws_bytes, (hipStream_t)stream);
 }
 
 int g4_attn_fwd_static(const g4_problem* p, const void* q, g4_layout ql, const void* k,
@@ -522,7 +527,7 @@ int g4_attn_fwd_static(const g4_problem* p, const void* q, g4_layout ql, const v
   }
   void* ws = nullptr;
   G4_TRY(scratch_for_stream((hipStream_t)stream, &ws));
-  return fwd_impl(p, q, ql, k, kl, v, vl, o, ol, lse, ws, (hipStream_t)stream);
+  return fwd_impl(p, q, ql, k, kl, v, vl, o, ol, lse, ws, need, (hipStream_t)stream);
 }
 
 static int fill_bwd(g4::BwdParams& a, const g4_problem* p, const void* q, g4_layout ql,

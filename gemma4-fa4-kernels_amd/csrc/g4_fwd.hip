@@ -12,6 +12,8 @@
 //   from the natural-layout V tile by transposing LDS reads.
 // K and V tiles are copied global -> LDS asynchronously (one 16-byte chunk per
 // lane) one tile ahead of the compute.
+#include <algorithm>
+
 #include "g4_kernels.h"
 
 namespace g4 {
@@ -342,6 +344,33 @@ struct FwdItem {
   }
 };
 
+// Item L of the rescaling pass after the wide kernel: 64 queries (tile qt) of
+// one head of sequence s, heads innermost.
+struct FixupItem {
+  static constexpr int kBM = 64;
+  int s, qt, qh;
+  __device__ __forceinline__ FixupItem(const FwdParams& a, int L) {
+    const int hq = a.p.num_q_heads;
+    qh = L % hq;
+    qt = L / hq % a.ntq;
+    s = L / hq / a.ntq;
+  }
+  // Whether the wide kernel flagged a row group of these queries and KV head
+  // (raise_flags; the group's heads share their slots).
+  __device__ __forceinline__ bool flagged(const FwdParams& a) const {
+    const g4_problem& p = a.p;
+    const int lq = p.cu_seqlens_q ? p.cu_seqlens_q[s + 1] - p.cu_seqlens_q[s] : p.seqlen_q;
+    const int grp = p.num_q_heads / p.num_kv_heads;
+    const int nq32 = (p.seqlen_q + 31) / 32;
+    int any = 0;
+    for (int q32 = qt * 2; q32 < qt * 2 + 2 && q32 * 32 < lq; ++q32) {
+      const int* f = a.raise_flags + ((int64_t)s * nq32 + q32) * p.num_q_heads + qh / grp * grp;
+      for (int j = 0; j < grp; ++j) any |= f[j];
+    }
+    return any != 0;
+  }
+};
+
 // Workgroups of a forward grid of bm-query tiles; sets b->compact.  A packed
 // batch of 2..64 sequences enumerates only its tiles: at most
 // sum ceil(len / bm) <= (total_q + num_seqs (bm - 1)) / bm per head, against
@@ -368,7 +397,7 @@ static int64_t fwd_grid(FwdParams* b, int bm, bool allow_compact) {
 }
 
 // One work item L of the forward (one query tile of one head).
-// FIXUP: rerun only the 32-query groups the wide kernel flagged in raise_flags.
+// FIXUP: item L of the rescaling pass (FixupItem).
 // OCC: workgroups per CU the register budget is sized for.
 template <int D, int BN, int DSPLIT, int NQG, bool VDOUBLE, int META, bool FIXUP, int OCC>
 __device__ __forceinline__ void fwd_item(const FwdParams& a, char* smem_raw, int L) {
@@ -389,24 +418,25 @@ __device__ __forceinline__ void fwd_item(const FwdParams& a, char* smem_raw, int
 
   // ---- work item -------------------------------------------------------
   FwdItem it;
-  if (!it.decode(a, L, C::kBM)) return;
-  const int kvh = it.kvh, qh = it.qh, s = it.s;
-  const int qt = zigzag(it.local, it.nt);
+  int kvh, qh, s, qt;
+  if constexpr (FIXUP) {
+    const FixupItem f(a, L);
+    kvh = f.qh / (p.num_q_heads / p.num_kv_heads);
+    qh = f.qh;
+    s = f.s;
+    qt = f.qt;
+  } else {
+    if (!it.decode(a, L, C::kBM)) return;
+    kvh = it.kvh;
+    qh = it.qh;
+    s = it.s;
+    qt = zigzag(it.local, it.nt);
+  }
 
   ker.sq = resolve_seq(p, s);
   const Seq& sq = ker.sq;
   const int i0 = qt * C::kBM;
   if (i0 >= sq.lq) return;
-  if constexpr (FIXUP) {
-    const int nq32 = (p.seqlen_q + 31) / 32;
-    bool need = false;
-#pragma unroll
-    for (int g = 0; g < NQG; ++g) {
-      const int q32 = i0 / 32 + g;
-      if (q32 < nq32) need |= a.raise_flags[((int64_t)s * nq32 + q32) * p.num_q_heads + qh] != 0;
-    }
-    if (!need) return;
-  }
   const int off = sq.lk - sq.lq;  // query i sits at key position i + off
   ker.a0 = i0 + off;
   const int a_last_valid = min(i0 + C::kBM, sq.lq) - 1 + off;
@@ -527,6 +557,7 @@ __device__ __forceinline__ void fwd_item(const FwdParams& a, char* smem_raw, int
 template <int D, int BN, int DSPLIT, int NQG, bool VDOUBLE, int META, bool FIXUP = false,
           int OCC = 1>
 __global__ void __launch_bounds__(NQG * DSPLIT * 64, OCC) fwd_kernel(FwdParams a) {
+  using C = FwdCfg<D, BN, DSPLIT, NQG, VDOUBLE>;
   extern __shared__ __attribute__((aligned(16))) char smem_raw[];
   if constexpr (META == 3 && !FIXUP) {
     // Second document pass with the first pass's list: the listed items,
@@ -540,6 +571,25 @@ __global__ void __launch_bounds__(NQG * DSPLIT * 64, OCC) fwd_kernel(FwdParams a
       const int L = listed ? __builtin_amdgcn_readfirstlane(a.doc_list[t])
                            : FwdItem::of_block(a);
       fwd_item<D, BN, DSPLIT, NQG, VDOUBLE, META, FIXUP, OCC>(a, smem_raw, L);
+    }
+  } else if constexpr (FIXUP) {
+    // Rescaling pass: items blockIdx.x, + gridDim.x, ... tested 64 at a time,
+    // one per lane (every wave the same), the flagged ones run.  Flags are
+    // rare, so the pass is its test: one workgroup per item spent 119 us on
+    // 33792 workgroups of 32 packed sequences (32768 tokens).
+    static_assert(C::kBM == FixupItem::kBM, "rescaling tiles");
+    const int n = a.num_seqs * a.ntq * a.p.num_q_heads;
+    const int lane = threadIdx.x & 63;
+    for (int64_t base = blockIdx.x; base < n; base += (int64_t)64 * gridDim.x) {
+      const int64_t mine = base + (int64_t)lane * gridDim.x;
+      unsigned long long todo = __ballot(mine < n && FixupItem(a, (int)mine).flagged(a));
+      while (todo) {
+        const int b = __builtin_amdgcn_readfirstlane(__ffsll((long long)todo) - 1);
+        todo &= todo - 1;
+        barrier_lds();  // the previous item's LDS reads are done
+        fwd_item<D, BN, DSPLIT, NQG, VDOUBLE, META, FIXUP, OCC>(a, smem_raw,
+                                                                (int)(base + b * gridDim.x));
+      }
     }
   } else {
     fwd_item<D, BN, DSPLIT, NQG, VDOUBLE, META, FIXUP, OCC>(a, smem_raw, FwdItem::of_block(a));
@@ -754,8 +804,15 @@ static hipError_t launch_fwd_split(const FwdParams& a, hipStream_t stream) {
 // ===========================================================================
 // Software-pipelined forward for wide heads without key metadata.
 //
-// Four waves, one per SIMD, each owning 32 queries and the whole head dim, so
-// no partial scores are exchanged and one K / V tile serves 128 queries.  Per
+// A workgroup owns 128 query rows of one KV head: 128 / grp consecutive queries
+// with the grp query heads of its group, query-major (row r is query r / grp,
+// head r % grp).  Rows of fewer queries end closer to one causal end than 128
+// queries of one head do: with GQA 8 a tile walks on average half a key tile
+// past its rows' ends instead of two (1000 tokens: 16.1 key tiles a workgroup
+// against 18), and a chunk of 16 new tokens is one tile per KV head, not 32
+// nearly empty ones.
+// Four waves, one per SIMD, each owning 32 rows and the whole head dim, so
+// no partial scores are exchanged and one K / V tile serves 128 rows.  Per
 // key tile the loop runs two regions:
 //   A: S^T(t+1) = K(t+1) Q^T on MFMA, interleaved with the softmax of tile t
 //      (VALU) and with the async copies of K(t+2) and V(t+1);
@@ -768,8 +825,16 @@ static hipError_t launch_fwd_split(const FwdParams& a, hipStream_t stream) {
 // same m as long as their maximum stays below m + kRaiseLog2 (log2 units), so
 // P = exp2(s - m) <= 2^kRaiseLog2 is exact in fp32 and in bf16 range and O, l
 // stay far from fp32 overflow.  A row whose scores jump higher (by more than
-// kRaiseLog2 * ln 2 within the row) marks its 32-query group in raise_flags;
-// launch_fwd then reruns exactly those groups with the rescaling kernel.
+// kRaiseLog2 * ln 2 within the row) marks its wave's 32 rows in raise_flags;
+// launch_fwd then reruns the 64-query tiles of those rows with the rescaling
+// kernel.
+//
+// SPLIT: few query rows over a long cached prefix (500 new tokens after 12000
+// are 128 workgroups; 16 are 4) do not fill the GPU.  Each tile's key tiles are
+// then cut into kv_chunks equal chunks, one workgroup each, which write their
+// rows' unnormalised O, maximum and sum to the workspace for
+// merge_wide_kernel.  Chunk-major within a KV head, so that the workgroups of
+// an XCD walk the same keys.
 // ===========================================================================
 
 constexpr float kRaiseLog2 = 48.0f;
@@ -804,7 +869,7 @@ struct FwdWide {
   char G4_LDS* smem;
   Seq sq;
   int lane, wave, h32;
-  int a0, window, lo_w, hi_c;
+  int a0, a_last, window, lo_w, hi_c;  // positions of the tile's first / last query
   const __bf16* kbase;
   const __bf16* vbase;
   int64_t kstride, vstride;
@@ -834,7 +899,7 @@ struct FwdWide {
   // Softmax of one tile's raw scores (keys kb0 + ...) into bf16 P.
   __device__ __forceinline__ void softmax(f32x16& s, int kb0, bf16x8 (&pb)[2]) {
     const bool full = (kb0 + BN <= sq.lk) && (kb0 + BN - 1 <= a0) &&
-                      (window <= 0 || kb0 > a0 + C::kBM - 1 - window);
+                      (window <= 0 || kb0 > a_last - window);
     if (!full) {
 #pragma unroll
       for (int r = 0; r < 16; ++r) {
@@ -863,7 +928,64 @@ struct FwdWide {
   }
 };
 
+// Query tile at rank r among a sequence's n: zigzag over groups of 8 adjacent
+// tiles (heaviest first within a group), the group that may be short first.
+// An XCD's run of ranks then holds light and heavy tiles alike, and neighbours
+// cost about the same: the hardware deals workgroups to the shader engines of
+// an XCD in turn, and with heavy and light tiles alternating one by one half of
+// the engines took the heavy ones while the others waited (32 packed sequences,
+// 32768 tokens: CUs busy 71% of the launch, 2.81 ms; in groups, and with the
+// rows leaving through LDS, 2.16 ms).
+constexpr int kWideGroup = 8;
+__device__ __forceinline__ int wide_tile(int r, int n) {
+  const int ng = (n + kWideGroup - 1) / kWideGroup;
+  const int first = n - (ng - 1) * kWideGroup;  // tiles of the last group
+  if (r < first) return n - 1 - r;
+  const int x = r - first;
+  return zigzag(1 + x / kWideGroup, ng) * kWideGroup + kWideGroup - 1 - x % kWideGroup;
+}
+
+// Query tile of a wide workgroup: KV head kvh, key chunk, sequence s, tile qt.
+struct WideItem {
+  int kvh, chunk, s, qt;
+  int row_tile;  // (KV head, tile) index of the partial rows
+  __device__ __forceinline__ bool decode(const FwdParams& a, int L, int queries) {
+    SeqTiles tiles;
+    if (a.compact) tiles.init(a.p.cu_seqlens_q, a.num_seqs, queries);
+    const int per_kvh = a.compact ? tiles.total : a.num_seqs * a.ntq;
+    const int n = a.kv_chunks;
+    kvh = L / (per_kvh * n);
+    if (kvh >= a.p.num_kv_heads) return false;
+    chunk = L / per_kvh % n;
+    const int rank = L % per_kvh;
+    row_tile = kvh * per_kvh + rank;
+    int local, nt;
+    if (a.compact) {
+      tiles.find(rank, s, local, nt);
+    } else {
+      s = rank / a.ntq;
+      local = rank % a.ntq;
+      nt = a.ntq;
+    }
+    qt = wide_tile(local, nt);
+    return true;
+  }
+};
+
+// Raise-flag slot of the 32-row wave whose first query is q (a multiple of
+// 32 / grp): the grp waves of a 32-query group take the group's head slots.
+__device__ __forceinline__ int64_t raise_slot(const g4_problem& p, int s, int q, int kvh,
+                                              int grp) {
+  const int nq32 = (p.seqlen_q + 31) / 32;
+  return ((int64_t)s * nq32 + q / 32) * p.num_q_heads + kvh * grp + q % 32 * grp / 32;
+}
+
+// Floats of a chunk's partial rows: 128 x D of O in register order (per wave,
+// 1 KB per store), then the rows' maximum and sum.
 template <int D>
+constexpr int64_t kWidePartFloats = 128 * D + 256;
+
+template <int D, bool SPLIT>
 __global__ void __launch_bounds__(256, 1) fwd_wide_kernel(FwdParams a) {
   using K = FwdWide<D>;
   using C = typename K::C;
@@ -878,25 +1000,34 @@ __global__ void __launch_bounds__(256, 1) fwd_wide_kernel(FwdParams a) {
   ker.h32 = ker.lane >> 5;
   const int l32 = ker.lane & 31;
 
-  const int L = FwdItem::of_block(a);
-  FwdItem it;
-  if (!it.decode(a, L, C::kBM)) return;
-  const int kvh = it.kvh, qh = it.qh, s = it.s;
-  const int qt = zigzag(it.local, it.nt);
+  const int L = a.desc_order ? xcd_remap_desc(blockIdx.x, gridDim.x, kWideGroup)
+                             : xcd_remap(blockIdx.x, gridDim.x);
+  const int grp = p.num_q_heads / p.num_kv_heads;
+  const int gsh = __builtin_ctz(grp);  // grp is 1, 2, 4 or 8
+  const int queries = C::kBM >> gsh;   // of a tile
+  WideItem it;
+  if (!it.decode(a, L, queries)) return;
+  const int kvh = it.kvh, s = it.s;
 
   ker.sq = resolve_seq(p, s);
   const Seq& sq = ker.sq;
-  const int i0 = qt * C::kBM;
+  const int i0 = it.qt * queries;
   if (i0 >= sq.lq) return;
   const int off = sq.lk - sq.lq;
   ker.a0 = i0 + off;
-  const int a_last_valid = min(i0 + C::kBM, sq.lq) - 1 + off;
+  ker.a_last = ker.a0 + queries - 1;
+  const int a_last_valid = min(i0 + queries, sq.lq) - 1 + off;
   ker.window = p.window;
 
   int klo, khi;
   query_tile_key_range(ker.a0, a_last_valid, sq.lk, p.window, -1, klo, khi);
-  const int t_first = klo / BN;
-  const int ntiles = (khi + BN - 1) / BN - t_first;
+  int t_first = klo / BN;
+  int ntiles = (khi + BN - 1) / BN - t_first;
+  if constexpr (SPLIT) {
+    const int lo = ntiles * it.chunk / a.kv_chunks;
+    ntiles = ntiles * (it.chunk + 1) / a.kv_chunks - lo;
+    t_first += lo;
+  }
 
   ker.kbase = a.k + tok_off(sq, s, sq.ktok, 0, a.kl) + (int64_t)kvh * a.kl.head_stride;
   ker.vbase = a.v + tok_off(sq, s, sq.ktok, 0, a.vl) + (int64_t)kvh * a.vl.head_stride;
@@ -907,7 +1038,9 @@ __global__ void __launch_bounds__(256, 1) fwd_wide_kernel(FwdParams a) {
   ker.kcp.init(ker.kstride, ker.wave, ker.lane);
   ker.vcp.init(ker.vstride, ker.wave, ker.lane);
 
-  const int my_i = i0 + ker.wave * 32 + l32;
+  const int w_q = i0 + ((ker.wave * 32) >> gsh);  // the wave's first query
+  const int my_i = w_q + (l32 >> gsh);
+  const int qh = kvh * grp + (l32 & (grp - 1));
   const int my_a = my_i + off;
   const bool q_valid = my_i < sq.lq;
   ker.lo_w = p.window > 0 ? my_a - p.window + 1 : -0x40000000;
@@ -973,46 +1106,226 @@ __global__ void __launch_bounds__(256, 1) fwd_wide_kernel(FwdParams a) {
     s_cur = s_nxt;
   }
 
-  // Every 32-query group reports whether its rows need the rescaling pass.
-  const int q32 = i0 / 32 + ker.wave;
-  const int nq32 = (p.seqlen_q + 31) / 32;
   const bool raise_any = __ballot(ker.raise && q_valid) != 0;
-  if (ker.lane == 0 && q32 < nq32)
-    a.raise_flags[((int64_t)s * nq32 + q32) * p.num_q_heads + qh] = raise_any ? 1 : 0;
-
   const float l_tot = ker.l_run + wave_xor32(ker.l_run);
-  const float inv = l_tot > 0.f ? 1.f / l_tot : 0.f;
-  if (q_valid) {
-    __bf16* orow = a.o + tok_off(sq, s, sq.qtok, my_i, a.ol) + (int64_t)qh * a.ol.head_stride;
+  if constexpr (SPLIT) {
+    float* part = a.part + ((int64_t)it.row_tile * a.kv_chunks + it.chunk) * kWidePartFloats<D>;
+    f32x4* po = (f32x4*)part + ker.wave * (K::kNB * 4 * 64) + ker.lane;
 #pragma unroll
-    for (int b = 0; b < K::kNB; ++b) {
+    for (int b = 0; b < K::kNB; ++b)
 #pragma unroll
       for (int r4 = 0; r4 < 4; ++r4) {
-        const int d = b * 32 + 8 * r4 + 4 * ker.h32;
-        const f32x16& acc = ker.o_acc[b];
-        bf16x4 v = {(__bf16)(acc[r4 * 4] * inv), (__bf16)(acc[r4 * 4 + 1] * inv),
-                    (__bf16)(acc[r4 * 4 + 2] * inv), (__bf16)(acc[r4 * 4 + 3] * inv)};
-        *(bf16x4*)(orow + d) = v;
+        const f32x16& x = ker.o_acc[b];
+        po[(b * 4 + r4) * 64] = f32x4{x[r4 * 4], x[r4 * 4 + 1], x[r4 * 4 + 2], x[r4 * 4 + 3]};
       }
-    }
     if (ker.h32 == 0) {
-      a.lse[lse_off(p, sq, s, qh, my_i)] =
-          l_tot > 0.f ? (ker.m_run + fast_log2(l_tot)) * kLn2 : kNegInf;
+      // (a sum of -1 marks the wave's rows for the rescaling pass)
+      float* ml = part + 128 * D + 2 * (ker.wave * 32 + l32);
+      ml[0] = ker.m_run;
+      ml[1] = raise_any ? -1.f : l_tot;
+    }
+    return;
+  }
+
+  // Every wave reports whether its rows need the rescaling pass; the last
+  // tile also clears the slots of its 32-query group past the tile.
+  if (ker.lane == 0 && w_q / 32 * 32 < sq.lq)
+    a.raise_flags[raise_slot(p, s, w_q, kvh, grp)] = raise_any ? 1 : 0;
+  const int i1 = i0 + queries;
+  if (i1 >= sq.lq && i1 % 32 != 0 && tid < grp && tid >= i1 % 32 * grp / 32)
+    a.raise_flags[raise_slot(p, s, i1 / 32 * 32, kvh, grp) + tid] = 0;
+
+  // The rows leave as whole lines through LDS (a lane's accumulators are one
+  // row's 8-byte runs): each wave stages its 32 rows in a quarter of the tile
+  // area, 16-byte chunks swizzled by row.  (Stored as they lie, an item spent
+  // 9-10 us after its loop; a 20-tile item's loop takes 40.)
+  const float inv = l_tot > 0.f ? 1.f / l_tot : 0.f;
+  static_assert(C::kNW * 32 * D * 2 <= C::kLdsBytes, "staged rows");
+  barrier_lds();  // every wave is done with the last tiles
+  char G4_LDS* stage = ker.smem + ker.wave * 32 * D * 2;
+#pragma unroll
+  for (int b = 0; b < K::kNB; ++b)
+#pragma unroll
+    for (int r4 = 0; r4 < 4; ++r4) {
+      const f32x16& acc = ker.o_acc[b];
+      *(bf16x4 G4_LDS*)(stage + l32 * D * 2 + ((b * 4 + r4) ^ (l32 & 15)) * 16 + 8 * ker.h32) =
+          bf16x4{(__bf16)(acc[r4 * 4] * inv), (__bf16)(acc[r4 * 4 + 1] * inv),
+                 (__bf16)(acc[r4 * 4 + 2] * inv), (__bf16)(acc[r4 * 4 + 3] * inv)};
+    }
+  if (q_valid && ker.h32 == 0)
+    a.lse[lse_off(p, sq, s, qh, my_i)] =
+        l_tot > 0.f ? (ker.m_run + fast_log2(l_tot)) * kLn2 : kNegInf;
+#pragma unroll 8
+  for (int r = 0; r < 32; ++r) {
+    const int i = w_q + (r >> gsh);
+    if (i >= sq.lq) break;
+    __bf16* orow = a.o + tok_off(sq, s, sq.qtok, i, a.ol) +
+                   (int64_t)(kvh * grp + (r & (grp - 1))) * a.ol.head_stride;
+    static_assert(D * 2 == 64 * 16, "one 16-byte chunk per lane and row");
+    *(bf16x8*)(orow + ker.lane * 8) =
+        *(const bf16x8 G4_LDS*)(stage + r * D * 2 + (ker.lane ^ (r & 15)) * 16);
+  }
+}
+
+// O and LSE of a split tile's rows from its chunks.  Workgroup (tile, wave of
+// 32 rows, quarter of the head dim): a thread keeps one row (its lane's), so
+// the chunks' weights 2^(m_c - M) are formed once per thread; the partials are
+// read in the order they were written (1 KB per wave instruction) and the
+// rows leave through LDS.
+template <int D>
+__global__ void __launch_bounds__(256) merge_wide_kernel(FwdParams a) {
+  using C = WideCfg<D>;
+  constexpr int kCols = D / 4;              // columns of a workgroup
+  constexpr int kPitch = kCols * 2 + 16;    // bytes of a staged row
+  __shared__ __attribute__((aligned(16))) char stage[32 * kPitch];
+  const g4_problem& p = a.p;
+  const int grp = p.num_q_heads / p.num_kv_heads;
+  const int gsh = __builtin_ctz(grp);
+  const int queries = C::kBM >> gsh;
+  const int n = a.kv_chunks;
+  const int quarter = blockIdx.x & 3, w = (blockIdx.x >> 2) & 3;
+  FwdParams one = a;  // the tile as the unsplit grid orders it
+  one.kv_chunks = 1;
+  WideItem it;
+  if (!it.decode(one, blockIdx.x >> 4, queries)) return;
+  const Seq sq = resolve_seq(p, it.s);
+  const int i0 = it.qt * queries;
+  if (i0 >= sq.lq) return;
+  const int w_q = i0 + ((w * 32) >> gsh);
+  const int tid = threadIdx.x, l32 = tid & 31, h32 = (tid >> 5) & 1, sub = tid >> 6;
+  const int my_i = w_q + (l32 >> gsh);
+  const int qh = it.kvh * grp + (l32 & (grp - 1));
+
+  const float* part = a.part + (int64_t)it.row_tile * n * kWidePartFloats<D>;
+  const float* ml = part + 128 * D + 2 * (w * 32 + l32);
+  float mx = kNegInf;
+  bool raise = false;
+  for (int c = 0; c < n; ++c) {
+    const float m = ml[c * kWidePartFloats<D>], l = ml[c * kWidePartFloats<D> + 1];
+    raise |= l < 0.f;
+    if (l > 0.f) mx = fmaxf(mx, m);
+  }
+  const bool raise_any = __ballot(raise) != 0;
+  if (quarter == 0 && tid == 0 && w_q / 32 * 32 < sq.lq)
+    a.raise_flags[raise_slot(p, it.s, w_q, it.kvh, grp)] = raise_any ? 1 : 0;
+  const int i1 = i0 + queries;
+  if (quarter == 0 && w == 0 && i1 >= sq.lq && i1 % 32 != 0 && tid < grp &&
+      tid >= i1 % 32 * grp / 32)
+    a.raise_flags[raise_slot(p, it.s, i1 / 32 * 32, it.kvh, grp) + tid] = 0;
+  if (w_q >= sq.lq || raise_any) return;  // no such rows, or written by the rescaling pass
+
+  // this workgroup's 32-column blocks of the wave's register-order partial
+  constexpr int kB = D / 32 / 4;  // blocks
+  static_assert(kB * 4 * 64 == 4 * 256, "four 16-byte loads per thread and chunk");
+  const f32x4* src = (const f32x4*)part + (w * (D / 32) + quarter * kB) * 4 * 64 + tid;
+  f32x4 acc[4] = {};
+  float l = 0.f;
+#pragma unroll 4
+  for (int c = 0; c < n; ++c) {
+    const float lc = ml[c * kWidePartFloats<D> + 1];
+    const float wt = lc > 0.f ? fast_exp2(ml[c * kWidePartFloats<D>] - mx) : 0.f;
+    l += wt * lc;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) acc[i] += wt * src[c * (kWidePartFloats<D> / 4) + i * 256];
+  }
+  const float inv = l > 0.f ? 1.f / l : 0.f;
+  // element i of a thread: block i, register group sub, row l32, columns
+  // 32 i + 8 sub + 4 h32 .. of the quarter
+#pragma unroll
+  for (int i = 0; i < 4; ++i)
+    *(bf16x4*)(stage + l32 * kPitch + (32 * i + 8 * sub + 4 * h32) * 2) =
+        bf16x4{(__bf16)(acc[i][0] * inv), (__bf16)(acc[i][1] * inv), (__bf16)(acc[i][2] * inv),
+               (__bf16)(acc[i][3] * inv)};
+  if (quarter == 0 && tid < 32 && my_i < sq.lq)
+    a.lse[lse_off(p, sq, it.s, qh, my_i)] = l > 0.f ? (mx + fast_log2(l)) * kLn2 : kNegInf;
+  __syncthreads();
+  const int row = tid >> 3;
+  const int oi = w_q + (row >> gsh);
+  if (oi >= sq.lq) return;
+  __bf16* orow = a.o + tok_off(sq, it.s, sq.qtok, oi, a.ol) +
+                 (int64_t)(it.kvh * grp + (row & (grp - 1))) * a.ol.head_stride + quarter * kCols;
+#pragma unroll
+  for (int i = 0; i < kCols / 64; ++i) {
+    const int c = (tid & 7) + 8 * i;
+    *(bf16x8*)(orow + c * 8) = *(const bf16x8*)(stage + row * kPitch + c * 16);
+  }
+}
+
+// Tiles per KV head of a wide launch's grid (an upper bound for packed
+// sequences): see fwd_grid.
+static int64_t wide_tiles(const g4_problem& p, int queries, int* compact) {
+  int64_t tiles = (int64_t)p.num_seqs * ((p.seqlen_q + queries - 1) / queries);
+  *compact = 0;
+  if (p.cu_seqlens_q != nullptr && p.num_seqs > 1 && p.num_seqs <= 64) {
+    const int64_t bound = (p.total_q + (int64_t)p.num_seqs * (queries - 1)) / queries;
+    if (bound < tiles) {
+      tiles = bound;
+      *compact = 1;
     }
   }
+  return tiles;
+}
+
+// Key chunks per query tile of the wide forward: 1 (no split) or the count
+// whose rounds of workgroups over the 256 CUs are shortest, in key tiles of one
+// workgroup's walk: (chunk + kSetup) per round, plus the merge (its launch and
+// the partials written and read at about 4 TB/s, a key tile taking 1.2 us).
+// At least kMinTiles key tiles a chunk.
+int wide_chunks(const g4_problem& p) {
+  if (p.head_dim != 512 || (p.vision_ids != nullptr && p.bidirectional_vision) ||
+      p.document_ids != nullptr)
+    return 1;
+  constexpr int kSetup = 6, kMinTiles = 8, kCus = 256;
+  int compact;
+  const int64_t items =
+      wide_tiles(p, 128 / (p.num_q_heads / p.num_kv_heads), &compact) * p.num_kv_heads;
+  const int64_t range = p.window > 0
+                            ? std::min<int64_t>(p.seqlen_k, (int64_t)p.window + 128)
+                            : p.seqlen_k;
+  const int64_t nt = (range + 31) / 32;
+  int best = 1;
+  double best_cost = 0.9 * (double)((items + kCus - 1) / kCus) * (nt + kSetup);
+  for (int64_t n = 2; n <= 64 && n * kMinTiles <= nt && n * items <= 4 * kCus; ++n) {
+    const double cost = (double)((items * n + kCus - 1) / kCus) * ((nt + n - 1) / n + kSetup) + 5 +
+                        (double)(items * n) * kWidePartFloats<512> * 8 / 4e6 / 1.2;
+    if (cost < best_cost) {
+      best_cost = cost;
+      best = (int)n;
+    }
+  }
+  return best;
+}
+size_t wide_split_bytes(const g4_problem& p) {
+  const int n = wide_chunks(p);
+  if (n == 1) return 0;
+  int compact;
+  const int64_t tiles = wide_tiles(p, 128 / (p.num_q_heads / p.num_kv_heads), &compact);
+  return (size_t)tiles * p.num_kv_heads * n * kWidePartFloats<512> * 4;
 }
 
 template <int D>
 static hipError_t launch_fwd_wide(const FwdParams& a, hipStream_t stream) {
   using C = WideCfg<D>;
-  static LdsAttr attr;
-  hipError_t e = attr.ensure((const void*)fwd_wide_kernel<D>, C::kLdsBytes);
-  if (e != hipSuccess) return e;
   FwdParams b = a;
-  const int64_t nblocks = fwd_grid(&b, C::kBM, true);
+  const int grp = a.p.num_q_heads / a.p.num_kv_heads;
+  const int queries = C::kBM / grp;
+  b.ntq = (a.p.seqlen_q + queries - 1) / queries;
+  const int64_t tiles = wide_tiles(a.p, queries, &b.compact) * a.p.num_kv_heads;
+  const bool split = a.part != nullptr;
+  b.kv_chunks = split ? wide_chunks(a.p) : 1;
+  const int64_t nblocks = tiles * b.kv_chunks;
   if (nblocks <= 0) return hipSuccess;
-  hipLaunchKernelGGL(fwd_wide_kernel<D>, dim3((unsigned)nblocks), dim3(C::kNT), C::kLdsBytes,
-                     stream, b);
+  // heaviest first within each XCD (xcd_remap_desc): whole groups of ranks, and
+  // group parity = parity within the sequence
+  b.desc_order = !b.compact && b.ntq % (2 * kWideGroup) == 0 && nblocks % (16 * kWideGroup) == 0;
+  void (*kern)(FwdParams) = split ? fwd_wide_kernel<D, true> : fwd_wide_kernel<D, false>;
+  static LdsAttr attr[2];
+  hipError_t e = attr[split].ensure((const void*)kern, C::kLdsBytes);
+  if (e != hipSuccess) return e;
+  hipLaunchKernelGGL(kern, dim3((unsigned)nblocks), dim3(C::kNT), C::kLdsBytes, stream, b);
+  e = hipGetLastError();
+  if (e != hipSuccess || !split) return e;
+  hipLaunchKernelGGL(merge_wide_kernel<D>, dim3((unsigned)(tiles * 16)), dim3(256), 0, stream, b);
   return hipGetLastError();
 }
 
@@ -1021,6 +1334,9 @@ static int meta_kind(const g4_problem& p) {
   return ((p.vision_ids != nullptr && p.bidirectional_vision) ? 1 : 0) |
          (p.document_ids != nullptr ? 2 : 0);
 }
+
+// Workgroups of the rescaling pass: one per CU.
+constexpr int kFixupGrid = 256;
 
 // meta < 0: the problem's own metadata kinds; doc_pass: see FwdParams.
 template <int D, int BN, int DSPLIT, int NQG, bool VDOUBLE, int OCC = 1>
@@ -1032,8 +1348,9 @@ static hipError_t launch_fwd_cfg(const FwdParams& a, hipStream_t stream, bool fi
       meta == 1   ? fwd_kernel<D, BN, DSPLIT, NQG, VDOUBLE, 1, false, OCC>
       : meta == 2 ? fwd_kernel<D, BN, DSPLIT, NQG, VDOUBLE, 2, false, OCC>
       : meta == 3 ? fwd_kernel<D, BN, DSPLIT, NQG, VDOUBLE, 3, false, OCC>
-      : fixup     ? fwd_kernel<D, BN, DSPLIT, NQG, VDOUBLE, 0, true, OCC>
                   : fwd_kernel<D, BN, DSPLIT, NQG, VDOUBLE, 0, false, OCC>;
+  if constexpr (D == 512)
+    if (fixup) kern = fwd_kernel<D, BN, DSPLIT, NQG, VDOUBLE, 0, true, OCC>;
   const int variant = fixup ? 4 : meta;
   static LdsAttr attr[5];
   hipError_t e = attr[variant].ensure((const void*)kern, C::kLdsBytes);
@@ -1043,6 +1360,7 @@ static hipError_t launch_fwd_cfg(const FwdParams& a, hipStream_t stream, bool fi
   // (the fixup pass and the listed second document pass decode full-grid indices)
   int64_t nblocks = fwd_grid(&b, C::kBM, !fixup && doc_pass != 2);
   if (nblocks <= 0) return hipSuccess;
+  if (fixup) nblocks = std::min<int64_t>(nblocks, kFixupGrid);
   if (doc_pass == 2 && a.doc_list != nullptr) {
     // the first pass's list, over at most one resident grid
     static PersistentGrid grid;

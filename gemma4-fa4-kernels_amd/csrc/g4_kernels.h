@@ -19,7 +19,9 @@ struct FwdParams {
   const int* span_hi;  // per K-stream token: last position of its vision span (or itself)
   int num_seqs;
   int ntq;             // query tiles per sequence (set by the launcher)
-  int* raise_flags;    // per (seq, 32-query group, head): rows the fast pass cannot finish
+  // Per (seq, 32-query group, head slot): row groups the fast pass cannot
+  // finish; the group's waves of the wide kernel take its KV head's slots.
+  int* raise_flags;
   // Split of a problem with document IDs over two launches (set by the
   // launcher): 0 every workgroup; 1 only workgroups whose queries and visited
   // keys share one document (their document test is dropped); 2 the others.
@@ -41,6 +43,9 @@ struct FwdParams {
   // partial rows (unnormalised O, running maximum and sum) go to `part`
   // before a merge launch.  0: the regular forward.
   int split_chunks, split_keys;
+  // Wide head-dim 512 forward: key chunks per query tile (set by the launcher;
+  // 1 unless `part` holds the chunks' partial rows).
+  int kv_chunks;
   float* part;
 };
 
@@ -200,6 +205,10 @@ size_t acc_bytes(const g4_problem& p);
 // Split-key forward: the number of key chunks per (sequence, KV head), 0 when
 // the problem takes the regular forward; *keys receives the keys per chunk.
 int split_chunks(const g4_problem& p, int* keys);
+// Wide head-dim 512 forward: key chunks per query tile (1: not split) and the
+// workspace bytes of their partial rows.
+int wide_chunks(const g4_problem& p);
+size_t wide_split_bytes(const g4_problem& p);
 // Workspace bytes of its partial rows (0 when not split).
 size_t split_bytes(const g4_problem& p);
 // Split dK/dV launch: parts (one per CU of the MI355X), floats of one partial

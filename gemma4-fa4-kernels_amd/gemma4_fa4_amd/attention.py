@@ -602,6 +602,19 @@ class _Plan:
                 nbytes = max(nbytes, split)
         return torch.empty(nbytes, dtype=torch.uint8, device=device)
 
+    def _forward_workspace_bytes(self, prob: G4Problem, device) -> int:
+        """The forward's workspace, with room to split its keys where that pays.
+
+        The partial rows (g4_workspace_bytes phase 3, at most 256 MiB) are a
+        speed-up, not a need: taken only within 10% of the free HBM.
+        """
+        nbytes = self.workspace_bytes(0, prob)
+        if self.head_dim == 512 and self.seqlen_k >= 512:
+            split = self.workspace_bytes(3, prob)
+            if split > nbytes and split <= _recent_free_hbm(device) // 10:
+                return split
+        return nbytes
+
     def forward(self, q, k, v):
         try:
             lib = _lib.load()
@@ -610,7 +623,7 @@ class _Plan:
             lse = torch.empty(self.lse_shape(), dtype=torch.float32, device=q.device)
             # Most forwards need no workspace (no vision IDs at head dim 256): the
             # library takes NULL for a zero-byte workspace, so none is allocated.
-            ws_bytes = self.workspace_bytes(0, prob)
+            ws_bytes = self._forward_workspace_bytes(prob, q.device)
             ws = torch.empty(ws_bytes, dtype=torch.uint8, device=q.device) if ws_bytes else None
         except Exception:
             self._settle()  # an invalid cu_seqlens is reported first

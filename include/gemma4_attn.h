@@ -97,7 +97,11 @@ const char* g4_last_error(void);
  * evenly, 128 MiB for fp32 partial dK / dV tiles.  A backward given at least
  * that much cuts its dK / dV work into equal parts over the CUs and adds the
  * partials in a fixed order; dQ is bitwise the same, dK / dV differ by the
- * order of the fp32 sums.  Equal to phase 1 when the split would not pay. */
+ * order of the fp32 sums.  Equal to phase 1 when the split would not pay.
+ * Phase 3: phase 0 plus, for a head-dim 512 forward whose query rows do not
+ * fill the GPU over a long key range (a chunk of new tokens after a cached
+ * prefix), the partial rows of key chunks.  A forward given at least that much
+ * splits its keys and merges the chunks. */
 size_t g4_workspace_bytes(const g4_problem* p, int phase);
 
 /*
