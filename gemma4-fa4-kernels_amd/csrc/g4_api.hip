@@ -197,9 +197,16 @@ int fwd_impl(const g4_problem* p, const void* q, g4_layout ql, const void* k, g4
   g4::span_arrays(*p, ws, &a.span_lo, &a.span_hi);
   a.raise_flags = raise_flags_ptr(*p, ws);
   a.part = split_ptr(*p, ws);
-  if (a.part != nullptr)
+  if (a.part != nullptr) {
     a.split_chunks = g4::split_chunks(*p, &a.split_keys);
-  else if (const size_t wide = g4::wide_split_bytes(*p); wide && ws_bytes >= fwd_ws_bytes(*p) + wide)
+    const int parts = g4::decode_parts(*p);
+    if (parts && ws_bytes >= fwd_ws_bytes(*p) - g4::split_bytes(*p) + g4::decode_bytes(*p)) {
+      a.split_chunks = parts;
+      a.split_slots = parts + p->num_seqs * p->num_kv_heads;
+    }
+  }
+  if (const size_t wide = g4::wide_split_bytes(*p);
+      a.part == nullptr && wide && ws_bytes >= fwd_ws_bytes(*p) + wide)
     a.part = (float*)((char*)ws + fwd_ws_bytes(*p));
   if (unsigned* dl = fwd_doc_list_ptr(*p, ws)) {
     a.doc_list_n = dl;
@@ -408,6 +415,25 @@ int split_chunks(const g4_problem& p, int* keys) {
   if (keys != nullptr) *keys = (int)(per * 32);
   return (int)n;
 }
+// Decode with equal parts (head dim 512): as many as are resident at once (two
+// workgroups per CU), of at least two tiles.  At most 16 rows: a part's rows
+// are 2 KB each and a tile's K and V 64 KB, and with 32 rows the partials cost
+// more than the balance gains (4 queries over 8192 keys: 35 us against 32).
+int decode_parts(const g4_problem& p) {
+  if (p.head_dim != 512 || split_chunks(p, nullptr) == 0) return 0;
+  if (p.num_q_heads / p.num_kv_heads * p.seqlen_q > 16) return 0;
+  const int64_t range = p.window > 0 ? std::min<int64_t>(p.seqlen_k, (int64_t)p.window + p.seqlen_q)
+                                     : p.seqlen_k;
+  const int64_t tiles = (int64_t)p.num_seqs * p.num_kv_heads * ((range + 31) / 32 + 1);
+  return (int)std::max<int64_t>(1, std::min<int64_t>(512, tiles / 2));
+}
+size_t decode_bytes(const g4_problem& p) {
+  const int parts = decode_parts(p);
+  if (parts == 0) return 0;
+  const size_t rows = (size_t)(p.num_q_heads / p.num_kv_heads) * p.seqlen_q;
+  return align256(((size_t)parts + (size_t)p.num_seqs * p.num_kv_heads) * rows *
+                  (p.head_dim + 2) * 4);
+}
 // Split dK/dV launch (g4_dkdv_split.h) against the launch by whole key tiles
 // (head dim 512: pairs of tiles) on the 256 CUs, in steps of the longest chain
 // of one CU (about 2.2 us at head dim 512, 1.9 us at 256).
@@ -501,7 +527,10 @@ size_t g4_workspace_bytes(const g4_problem* p, int phase) {
   if (phase == 1) return bwd_ws_bytes(*p);
   if (phase == 2) return bwd_ws_bytes(*p) + g4::dkdv_split_bytes(*p);
   if (phase == 3)
-    return fwd_ws_bytes(*p) + (g4::split_bytes(*p) ? 0 : g4::wide_split_bytes(*p));
+    return fwd_ws_bytes(*p) +
+           (g4::split_bytes(*p) ? std::max(g4::decode_bytes(*p), g4::split_bytes(*p)) -
+                                      g4::split_bytes(*p)
+                                : g4::wide_split_bytes(*p));
   return fwd_ws_bytes(*p);
 }
 

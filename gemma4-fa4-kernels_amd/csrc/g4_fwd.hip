@@ -802,6 +802,431 @@ static hipError_t launch_fwd_split(const FwdParams& a, hipStream_t stream) {
 }
 
 // ===========================================================================
+// Decode at head dim 512 with equal parts.
+//
+// As the split-key forward above (32 rows of one KV head's group), but what
+// bounds a decode step is how evenly, and with how many bytes in flight, the CUs
+// read the cache.  So the key tiles of all (sequence, KV head) segments lie end
+// to end and part g of n takes the g-th equal run of them, whatever the
+// sequences' lengths, and two workgroups share a CU (one K and one V tile each
+// in LDS, 72 KB), one's copies in flight while the other computes.  A part
+// writes its rows' state over each segment it touches to slot g + segment, and
+// merge_decode_kernel combines a segment's slots.  Before / after, both
+// launches: 1 x 8192 keys 29.2 / 26.9 us, 1 x 131072 249 / 199, 16 x 4K-8K
+// 204 / 149 (5.1 TB/s), 16 x 8192 238 / 197, 32 x 1000 66 / 55.
+// (Measured and not kept: the next segment's first copies and queries issued
+// from the last tile's step, 16 x 8192 219 us: the step grows and spills.  At
+// head dim 256 no gain: 32 x 1024 110 us against 105, 16 x 700 40 against 39.)
+// ===========================================================================
+
+template <int D>
+struct DecodeCfg {
+  static constexpr int kNW = D / 256;  // waves, each a 256-wide head-dim slice
+  static constexpr int kBN = 32;
+  static constexpr int kCPR = D / 8;
+  static constexpr int kTile = kBN * D * 2;
+  static constexpr int kNC = 16;  // 16-deep S steps of a slice
+  static constexpr int kNB = 8;   // 32-wide O blocks of a slice
+  static constexpr int kLdsK = 0;
+  static constexpr int kLdsV = kTile;
+  static constexpr int kLdsX = 2 * kTile;  // partial S of each wave
+  static constexpr int kLdsBytes = kLdsX + (kNW > 1 ? kNW * 4096 : 0);
+};
+
+// The key tiles of the segments, end to end: sequence-major, KV head, tile.
+struct DecodeMap {
+  const g4_problem* p;
+  int total;  // tiles of all segments
+
+  struct Keys {
+    int first, n;  // tiles a sequence's queries reach
+  };
+  __device__ __forceinline__ Keys keys(int s) const {
+    int lq = p->seqlen_q, lk = p->seqlen_k;
+    if (p->cu_seqlens_q != nullptr) {
+      lq = p->cu_seqlens_q[s + 1] - p->cu_seqlens_q[s];
+      lk = p->cu_seqlens_k[s + 1] - p->cu_seqlens_k[s];
+    }
+    if (lq <= 0) return {0, 0};
+    int lo, hi;
+    query_tile_key_range(lk - lq, lk - 1, lk, p->window, -1, lo, hi);
+    return {lo / 32, hi > lo ? (hi + 31) / 32 - lo / 32 : 0};
+  }
+  __device__ __forceinline__ static int scan(int x) {
+    const int lane = __lane_id();
+#pragma unroll
+    for (int o = 1; o < 64; o <<= 1) {
+      const int y = __shfl_up(x, o, 64);
+      if (lane >= o) x += y;
+    }
+    return x;
+  }
+  __device__ __forceinline__ void init(const g4_problem& prob) {
+    p = &prob;
+    if (p->cu_seqlens_q == nullptr) {
+      total = keys(0).n * p->num_seqs * p->num_kv_heads;
+      return;
+    }
+    int sum = 0;
+    for (int s = __lane_id(); s < p->num_seqs; s += 64) sum += keys(s).n;
+    total = __builtin_amdgcn_readlane(scan(sum), 63) * p->num_kv_heads;
+  }
+  // Sequence s that holds position pos < total, and its first position.
+  __device__ __forceinline__ void find(int pos, int& s, int& start) const {
+    const int hkv = p->num_kv_heads;
+    if (p->cu_seqlens_q == nullptr) {
+      const int per = keys(0).n * hkv;
+      s = pos / per;
+      start = s * per;
+      return;
+    }
+    start = 0;
+    for (int base = 0; base < p->num_seqs; base += 64) {
+      const int mine = base + (int)__lane_id();
+      const int cnt = mine < p->num_seqs ? keys(mine).n * hkv : 0;
+      const int incl = scan(cnt) + start;
+      const int end = __builtin_amdgcn_readlane(incl, 63);
+      if (pos < end) {
+        const int at = __builtin_amdgcn_readfirstlane(__popcll(__ballot(incl <= pos)));
+        s = base + at;
+        start = __builtin_amdgcn_readlane(incl - cnt, at);
+        return;
+      }
+      start = end;
+    }
+    s = p->num_seqs;  // (pos >= total)
+  }
+  // First position of sequence s.
+  __device__ __forceinline__ int start_of(int s) const {
+    if (p->cu_seqlens_q == nullptr) return s * keys(0).n * p->num_kv_heads;
+    int sum = 0;
+    for (int t = __lane_id(); t < s; t += 64) sum += keys(t).n;
+    return __builtin_amdgcn_readlane(scan(sum), 63) * p->num_kv_heads;
+  }
+  // First position of part g of n.
+  __device__ __forceinline__ int bound(int g, int n) const {
+    return (int)((int64_t)total * g / n);
+  }
+  // The part of n that holds position pos.
+  __device__ __forceinline__ int part_of(int pos, int n) const {
+    int g = (int)((int64_t)pos * n / total);
+    while (bound(g + 1, n) <= pos) ++g;
+    while (bound(g, n) > pos) --g;
+    return g;
+  }
+};
+
+template <int D>
+struct DecodeKernel {
+  using C = DecodeCfg<D>;
+  using Copier = TileCopier<C::kCPR, C::kBN, C::kNW>;
+  static constexpr int kPer = Copier::kPer;  // copy instructions of a tile per wave
+  char G4_LDS* smem;
+  const FwdParams* a;
+  Seq sq;
+  int lane, dh, h32, r;
+  int off, lq, my_a;
+  const __bf16* kbase;
+  const __bf16* vbase;
+  RowReader<C::kCPR> krd;
+  TrReader<C::kCPR> vrd;
+  Copier kcp, vcp;
+  bf16x8 qf[C::kNC];
+  f32x16 o_acc[C::kNB];
+  float m_run, l_run;
+
+  __device__ __forceinline__ void issue(const Copier& cp, const __bf16* base, int64_t stride,
+                                        int row0, int lds) {
+    if (row0 + C::kBN <= sq.lk)
+      cp.issue(base + row0 * stride, smem + lds);
+    else
+      cp.issue_clamped(base + row0 * stride, stride, sq.lk - row0, smem + lds);
+  }
+  __device__ __forceinline__ void issue_k(int t) {
+    issue(kcp, kbase, a->kl.token_stride, t * C::kBN, C::kLdsK);
+  }
+  __device__ __forceinline__ void issue_v(int t) {
+    issue(vcp, vbase, a->vl.token_stride, t * C::kBN, C::kLdsV);
+  }
+
+  // Key tile t; its K and V copies are in flight (K issued first).
+  __device__ __forceinline__ void step(int t, bool more) {
+    const int kb0 = t * C::kBN;
+    vm_wait<kPer>();
+    barrier_lds();  // K(t) has landed in every wave
+    f32x16 sv = f32x16{};
+    __builtin_amdgcn_sched_barrier(0);
+    row_steps<C::kNC, 4>(krd, smem + C::kLdsK, sv, qf);
+    __builtin_amdgcn_sched_barrier(0);
+    if constexpr (C::kNW > 1) {
+      char G4_LDS* xb = smem + C::kLdsX;
+#pragma unroll
+      for (int q4 = 0; q4 < 4; ++q4)
+        *(f32x4 G4_LDS*)(xb + ((dh * 4 + q4) * 64 + lane) * 16) =
+            f32x4{sv[q4 * 4], sv[q4 * 4 + 1], sv[q4 * 4 + 2], sv[q4 * 4 + 3]};
+      barrier_lds();
+#pragma unroll
+      for (int q4 = 0; q4 < 4; ++q4) {
+        const f32x4 v = *(const f32x4 G4_LDS*)(xb + (((dh ^ 1) * 4 + q4) * 64 + lane) * 16);
+        // added in slice order, so that both slices hold the same scores
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          const float mine = sv[q4 * 4 + e];
+          sv[q4 * 4 + e] = dh == 0 ? mine + v[e] : v[e] + mine;
+        }
+      }
+    }
+    if (more) issue_k(t + 1);  // every wave is done with K(t)
+
+    const int window = a->p.window;
+    const bool full = kb0 + C::kBN <= sq.lk && kb0 + C::kBN - 1 <= off &&
+                      (window <= 0 || kb0 > off + lq - 1 - window);
+    if (!full) {
+      const int lo_w = window > 0 ? my_a - window + 1 : -0x40000000;
+      const int hi_c = min(my_a, sq.lk - 1);
+#pragma unroll
+      for (int e = 0; e < 16; ++e) {
+        const int j = kb0 + 8 * (e >> 2) + 4 * h32 + (e & 3);
+        sv[e] = j >= lo_w && j <= hi_c ? sv[e] : kNegInf;
+      }
+    }
+    float mx = sv[0];
+#pragma unroll
+    for (int e = 1; e < 16; ++e) mx = fmaxf(mx, sv[e]);
+    mx = fmaxf(mx, wave_xor32(mx)) * kLog2e;
+    const float m_new = mx > m_run + kRescaleLog2 ? mx : m_run;
+    const float m_use = m_new == kNegInf ? 0.f : m_new;
+    const float alpha = fast_exp2(m_run - m_use);
+    float rs = 0.f;
+    bf16x8 pb[2];
+#pragma unroll
+    for (int e = 0; e < 16; ++e) {
+      const float pv = fast_exp2(__builtin_fmaf(sv[e], kLog2e, -m_use));
+      rs += pv;
+      pb[e >> 3][e & 7] = (__bf16)pv;
+    }
+    l_run = l_run * alpha + rs;
+    m_run = m_new;
+    if (__ballot(alpha != 1.f)) {
+#pragma unroll
+      for (int b = 0; b < C::kNB; ++b) o_acc[b] *= alpha;
+    }
+    if (more)
+      vm_wait<kPer>();
+    else
+      vm_wait<0>();
+    barrier_lds();  // V(t) has landed in every wave
+    __builtin_amdgcn_sched_barrier(0);
+    acc_steps<C::kNB, 4>(vrd, smem + C::kLdsV, pb, o_acc);
+    __builtin_amdgcn_sched_barrier(0);
+    barrier_lds();  // every wave is done with V(t)
+    if (more) issue_v(t + 1);
+  }
+};
+
+template <int D>
+__global__ void __launch_bounds__(D / 4) fwd_decode_kernel(FwdParams a) {
+  using K = DecodeKernel<D>;
+  using C = typename K::C;
+  extern __shared__ __attribute__((aligned(16))) char smem_raw[];
+  const g4_problem& p = a.p;
+  K ker;
+  ker.smem = (char G4_LDS*)smem_raw;
+  ker.a = &a;
+  ker.lane = threadIdx.x & 63;
+  ker.dh = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  ker.h32 = ker.lane >> 5;
+  ker.r = ker.lane & 31;
+  ker.krd.init(ker.lane, ker.dh * 512);
+  ker.vrd.init(ker.lane, ker.dh * 512);
+  ker.kcp.init(a.kl.token_stride, ker.dh, ker.lane);
+  ker.vcp.init(a.vl.token_stride, ker.dh, ker.lane);
+  const int grp = p.num_q_heads / p.num_kv_heads;
+  const int rows = grp * p.seqlen_q;  // row stride of the partial slots
+
+  const int g = xcd_remap(blockIdx.x, gridDim.x);
+  DecodeMap map;
+  map.init(p);
+  const int n = min(a.split_chunks, map.total);  // (every part holds a tile)
+  if (g >= n) return;
+  int pos = map.bound(g, n);
+  const int end = map.bound(g + 1, n);
+  int s, start;
+  map.find(pos, s, start);
+  while (pos < end) {
+    const DecodeMap::Keys keys = map.keys(s);
+    if (keys.n == 0) {
+      ++s;
+      continue;
+    }
+    const int kvh = (pos - start) / keys.n;
+    const int t_lo = (pos - start) - kvh * keys.n;
+    const int t_hi = min(keys.n, t_lo + end - pos);
+    ker.sq = resolve_seq(p, s);
+    const Seq& sq = ker.sq;
+    ker.lq = sq.lq;
+    ker.off = sq.lk - sq.lq;
+    const bool valid = ker.r < grp * sq.lq;
+    const int qh = kvh * grp + (valid ? ker.r / sq.lq : 0);
+    const int qi = valid ? ker.r % sq.lq : 0;
+    ker.my_a = qi + ker.off;
+    ker.kbase = a.k + tok_off(sq, s, sq.ktok, 0, a.kl) + (int64_t)kvh * a.kl.head_stride;
+    ker.vbase = a.v + tok_off(sq, s, sq.ktok, 0, a.vl) + (int64_t)kvh * a.vl.head_stride;
+    const __bf16* qrow = a.q + tok_off(sq, s, sq.qtok, qi, a.ql) +
+                         (int64_t)qh * a.ql.head_stride + ker.dh * 256 + ker.h32 * 8;
+#pragma unroll
+    for (int cc = 0; cc < C::kNC; ++cc) ker.qf[cc] = ld_global16(qrow + cc * 16);
+    ker.issue_k(keys.first + t_lo);
+    ker.issue_v(keys.first + t_lo);
+#pragma unroll
+    for (int cc = 0; cc < C::kNC; ++cc) ker.qf[cc] = valid ? ker.qf[cc] : bf16x8{};
+#pragma unroll
+    for (int b = 0; b < C::kNB; ++b) ker.o_acc[b] = f32x16{};
+    ker.m_run = kNegInf;
+    ker.l_run = 0.f;
+    for (int t = t_lo; t < t_hi; ++t) ker.step(keys.first + t, t + 1 < t_hi);
+
+    // ---- this part's rows of the segment: slot g + segment -------------------
+    const float l_tot = ker.l_run + wave_xor32(ker.l_run);
+    if (valid) {
+      const int64_t row = ((int64_t)g + s * p.num_kv_heads + kvh) * rows + ker.r;
+      float* po = a.part + row * D;
+#pragma unroll
+      for (int b = 0; b < C::kNB; ++b)
+#pragma unroll
+        for (int r4 = 0; r4 < 4; ++r4) {
+          const int d = ker.dh * 256 + b * 32 + 8 * r4 + 4 * ker.h32;
+          const f32x16& x = ker.o_acc[b];
+          *(f32x4*)(po + d) = f32x4{x[r4 * 4], x[r4 * 4 + 1], x[r4 * 4 + 2], x[r4 * 4 + 3]};
+        }
+      if (ker.dh == 0 && ker.h32 == 0) {
+        float* ml = a.part + (int64_t)a.split_slots * rows * D + row * 2;
+        ml[0] = ker.m_run;
+        ml[1] = l_tot;
+      }
+    }
+    pos += t_hi - t_lo;
+    if (kvh + 1 == p.num_kv_heads && t_hi == keys.n) {
+      start += keys.n * p.num_kv_heads;
+      ++s;
+    }
+  }
+}
+
+// One workgroup per (sequence, KV head, row, Q-th of the head dim).  What
+// bounds it is the chain of loads (a part's rows come from other XCDs, about
+// 2 us each time): the parts' maxima and sums are read at once and their weights
+// kept in LDS, then every thread's share of the O rows is in flight together
+// (kP parts per load instruction of the workgroup), and the kP sums are added
+// in order.  128 parts of an 8K cache: 17 us when each wave walked every fourth
+// part, reading its maximum, sum and row one after the other; 6.2 us like this.
+// Q = 4 while the rows alone are fewer workgroups than CUs (16 sequences, 512
+// rows of about ten parts: Q = 4 12.8 us, Q = 1 9.0).
+template <int D, int Q>
+__global__ void __launch_bounds__(256) merge_decode_kernel(FwdParams a) {
+  constexpr int kCols = D / Q;          // columns of a workgroup
+  constexpr int kLanes = kCols / 4;     // 16-byte loads of one part's row
+  constexpr int kP = 256 / kLanes;      // parts per load instruction
+  constexpr int kMaxParts = 512;
+  __shared__ float wts[kMaxParts];
+  __shared__ float red_m[4], red_l[4];
+  __shared__ float stage[kP][kCols];
+  const g4_problem& p = a.p;
+  const int grp = p.num_q_heads / p.num_kv_heads;
+  const int rows = grp * p.seqlen_q;
+  const int quarter = blockIdx.x % Q;
+  const int seg = blockIdx.x / Q / rows, r = blockIdx.x / Q % rows;
+  const int s = seg / p.num_kv_heads, kvh = seg % p.num_kv_heads;
+  const Seq sq = resolve_seq(p, s);
+  if (r >= grp * sq.lq) return;
+  const int qh = kvh * grp + r / sq.lq, qi = r % sq.lq;
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  DecodeMap map;
+  map.init(p);
+  const int tiles = map.keys(s).n;
+  int g0 = 0, n = 0;
+  if (tiles > 0) {
+    const int first = map.start_of(s) + kvh * tiles;
+    const int parts = min(a.split_chunks, map.total);
+    g0 = map.part_of(first, parts);
+    n = min(map.part_of(first + tiles - 1, parts) - g0 + 1, kMaxParts);
+  }
+  const float* ml = a.part + (int64_t)a.split_slots * rows * D;
+  const int64_t row0 = ((int64_t)g0 + seg) * rows + r;  // part c: row0 + c * rows
+  constexpr int kOwn = kMaxParts / 256;
+  float m_c[kOwn], l_c[kOwn];
+  float mx = kNegInf;
+#pragma unroll
+  for (int i = 0; i < kOwn; ++i) {
+    const int c = tid + 256 * i;
+    m_c[i] = kNegInf;
+    l_c[i] = 0.f;
+    if (c < n) {
+      const float* e = ml + (row0 + (int64_t)c * rows) * 2;
+      m_c[i] = e[0];
+      l_c[i] = e[1];
+      // (a part without keys for this row wrote l = 0 and O = 0)
+      if (l_c[i] > 0.f) mx = fmaxf(mx, m_c[i]);
+    }
+  }
+#pragma unroll
+  for (int o = 32; o > 0; o >>= 1) mx = fmaxf(mx, __shfl_xor(mx, o, 64));
+  if (lane == 0) red_m[wave] = mx;
+  __syncthreads();
+  mx = fmaxf(fmaxf(red_m[0], red_m[1]), fmaxf(red_m[2], red_m[3]));
+  float l = 0.f;
+#pragma unroll
+  for (int i = 0; i < kOwn; ++i) {
+    const int c = tid + 256 * i;
+    const float w = l_c[i] > 0.f ? fast_exp2(m_c[i] - mx) : 0.f;
+    if (c < n) wts[c] = w;
+    l += w * l_c[i];
+  }
+#pragma unroll
+  for (int o = 32; o > 0; o >>= 1) l += __shfl_xor(l, o, 64);
+  if (lane == 0) red_l[wave] = l;
+  __syncthreads();
+  l = (red_l[0] + red_l[1]) + (red_l[2] + red_l[3]);
+  const int sub = tid / kLanes, col = tid % kLanes;
+  const float* po = a.part + row0 * D + quarter * kCols + col * 4;
+  f32x4 acc = {};
+#pragma unroll 16
+  for (int c = sub; c < n; c += kP) acc += wts[c] * *(const f32x4*)(po + (int64_t)c * rows * D);
+  *(f32x4*)&stage[sub][col * 4] = acc;
+  __syncthreads();
+  if (tid >= kLanes) return;
+  acc = f32x4{};
+#pragma unroll
+  for (int u = 0; u < kP; ++u) acc += *(const f32x4*)&stage[u][tid * 4];
+  const float inv = l > 0.f ? 1.f / l : 0.f;
+  __bf16* orow = a.o + tok_off(sq, s, sq.qtok, qi, a.ol) + (int64_t)qh * a.ol.head_stride +
+                 quarter * kCols;
+  *(bf16x4*)(orow + tid * 4) = bf16x4{(__bf16)(acc[0] * inv), (__bf16)(acc[1] * inv),
+                                      (__bf16)(acc[2] * inv), (__bf16)(acc[3] * inv)};
+  if (quarter == 0 && tid == 0)
+    a.lse[lse_off(p, sq, s, qh, qi)] = l > 0.f ? (mx + fast_log2(l)) * kLn2 : kNegInf;
+}
+
+template <int D>
+static hipError_t launch_fwd_decode(const FwdParams& a, hipStream_t stream) {
+  using C = DecodeCfg<D>;
+  static LdsAttr attr;
+  hipError_t e = attr.ensure((const void*)fwd_decode_kernel<D>, C::kLdsBytes);
+  if (e != hipSuccess) return e;
+  const int64_t rows = (int64_t)a.num_seqs * a.p.num_q_heads * a.p.seqlen_q;
+  hipLaunchKernelGGL(fwd_decode_kernel<D>, dim3((unsigned)a.split_chunks), dim3(C::kNW * 64),
+                     C::kLdsBytes, stream, a);
+  e = hipGetLastError();
+  if (e != hipSuccess) return e;
+  if (rows < 256)
+    hipLaunchKernelGGL((merge_decode_kernel<D, 4>), dim3((unsigned)(rows * 4)), dim3(256), 0,
+                       stream, a);
+  else
+    hipLaunchKernelGGL((merge_decode_kernel<D, 1>), dim3((unsigned)rows), dim3(256), 0, stream, a);
+  return hipGetLastError();
+}
+
+// ===========================================================================
 // Software-pipelined forward for wide heads without key metadata.
 //
 // A workgroup owns 128 query rows of one KV head: 128 / grp consecutive queries
@@ -1378,6 +1803,7 @@ __global__ void clear_list_kernel(unsigned* n) {
 }
 
 hipError_t launch_fwd(const FwdParams& a, hipStream_t stream) {
+  if (a.split_slots > 0) return launch_fwd_decode<512>(a, stream);
   if (a.split_chunks > 0) {
     if (a.p.head_dim == 256) return launch_fwd_split<256>(a, stream);
     if (a.p.head_dim == 512) return launch_fwd_split<512>(a, stream);

@@ -43,6 +43,9 @@ struct FwdParams {
   // partial rows (unnormalised O, running maximum and sum) go to `part`
   // before a merge launch.  0: the regular forward.
   int split_chunks, split_keys;
+  // Decode with equal parts (head dim 512): split_chunks parts, split_slots
+  // slots of partial rows.  0: chunks of split_keys keys.
+  int split_slots;
   // Wide head-dim 512 forward: key chunks per query tile (set by the launcher;
   // 1 unless `part` holds the chunks' partial rows).
   int kv_chunks;
@@ -211,6 +214,10 @@ int wide_chunks(const g4_problem& p);
 size_t wide_split_bytes(const g4_problem& p);
 // Workspace bytes of its partial rows (0 when not split).
 size_t split_bytes(const g4_problem& p);
+// Decode with equal parts: their number (0 when the problem takes the chunks
+// of split_chunks) and the workspace bytes of their slots of partial rows.
+int decode_parts(const g4_problem& p);
+size_t decode_bytes(const g4_problem& p);
 // Split dK/dV launch: parts (one per CU of the MI355X), floats of one partial
 // slot (the dK and dV of one key tile, 64 x 512 or 128 x 256 each), and the
 // workspace bytes of the slots: 0 when the launch by whole tiles is as good.

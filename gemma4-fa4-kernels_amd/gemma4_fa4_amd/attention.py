@@ -602,18 +602,24 @@ class _Plan:
                 nbytes = max(nbytes, split)
         return torch.empty(nbytes, dtype=torch.uint8, device=device)
 
-    def _forward_workspace_bytes(self, prob: G4Problem, device) -> int:
-        """The forward's workspace, with room to split its keys where that pays.
+    def _forward_workspace(self, prob: G4Problem, device):
+        """The forward's workspace (None when it needs none) and its size.
 
-        The partial rows (g4_workspace_bytes phase 3, at most 256 MiB) are a
-        speed-up, not a need: taken only within 10% of the free HBM.
+        Phase 3 of g4_workspace_bytes, with room to split the keys over every
+        CU, where that is more than the forward needs; when that much (at most
+        256 MiB) cannot be had, what it needs.
         """
         nbytes = self.workspace_bytes(0, prob)
-        if self.head_dim == 512 and self.seqlen_k >= 512:
+        if self.head_dim == 512:
             split = self.workspace_bytes(3, prob)
-            if split > nbytes and split <= _recent_free_hbm(device) // 10:
-                return split
-        return nbytes
+            if split > nbytes:
+                try:
+                    return torch.empty(split, dtype=torch.uint8, device=device), split
+                except torch.OutOfMemoryError:
+                    pass
+        # Most local forwards need no workspace (no vision IDs): the library
+        # takes NULL for a zero-byte workspace, so none is allocated.
+        return (torch.empty(nbytes, dtype=torch.uint8, device=device) if nbytes else None), nbytes
 
     def forward(self, q, k, v):
         try:
@@ -621,10 +627,7 @@ class _Plan:
             prob = self.problem()
             out = torch.empty(q.shape, dtype=q.dtype, device=q.device)
             lse = torch.empty(self.lse_shape(), dtype=torch.float32, device=q.device)
-            # Most forwards need no workspace (no vision IDs at head dim 256): the
-            # library takes NULL for a zero-byte workspace, so none is allocated.
-            ws_bytes = self._forward_workspace_bytes(prob, q.device)
-            ws = torch.empty(ws_bytes, dtype=torch.uint8, device=q.device) if ws_bytes else None
+            ws, ws_bytes = self._forward_workspace(prob, q.device)
         except Exception:
             self._settle()  # an invalid cu_seqlens is reported first
             raise

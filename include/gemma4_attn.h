@@ -98,10 +98,10 @@ const char* g4_last_error(void);
  * that much cuts its dK / dV work into equal parts over the CUs and adds the
  * partials in a fixed order; dQ is bitwise the same, dK / dV differ by the
  * order of the fp32 sums.  Equal to phase 1 when the split would not pay.
- * Phase 3: phase 0 plus, for a head-dim 512 forward whose query rows do not
- * fill the GPU over a long key range (a chunk of new tokens after a cached
- * prefix), the partial rows of key chunks.  A forward given at least that much
- * splits its keys and merges the chunks. */
+ * Phase 3: phase 0 plus, for a forward whose query rows do not fill the GPU
+ * over a long key range (a decode step; at head dim 512 a chunk of new tokens
+ * after a cached prefix), room for more partial rows.  A forward given at least
+ * that much splits its keys over all CUs and merges the parts. */
 size_t g4_workspace_bytes(const g4_problem* p, int phase);
 
 /*
@@ -114,8 +114,8 @@ size_t g4_workspace_bytes(const g4_problem* p, int phase);
  *   global V-slab pairs        src/gemma4_fa4/h100.py:1148-1190, 1320-1387, 1013-1036
  * One launch covers the full Dv (no V slabs).  Problems without key
  * metadata whose query rows per KV head (query heads of a group x Sq) fit 32,
- * over at least 256 keys (a decode step), split the keys into chunks over
- * the GPU and merge the chunks' partial rows (kept in the workspace, which
+ * over at least 256 keys (a decode step), split the keys into parts over
+ * the GPU and merge the parts' partial rows (kept in the workspace, which
  * g4_workspace_bytes counts): two launches.
  */
 int g4_attn_fwd(const g4_problem* p,
