@@ -637,9 +637,10 @@ int g4_attn_bwd_dkdv(const g4_problem* p, const void* q, g4_layout ql, const voi
   return G4_OK;
 }
 
-int g4_attn_bwd_dq(const g4_problem* p, const void* q, g4_layout ql, const void* k, g4_layout kl,
-                   const void* v, g4_layout vl, const void* dout, g4_layout dol, const float* lse,
-                   void* dq, g4_layout dql, void* ws, size_t ws_bytes, void* stream) {
+static int bwd_dq(const g4_problem* p, const void* q, g4_layout ql, const void* k, g4_layout kl,
+                  const void* v, g4_layout vl, const void* dout, g4_layout dol, const float* lse,
+                  void* dq, g4_layout dql, void* ws, size_t ws_bytes, bool after_delta,
+                  void* stream) {
   g_last_error.clear();
   G4_TRY(check_problem(p));
   G4_TRY(check_operand(q, ql, "q"));
@@ -656,9 +657,16 @@ int g4_attn_bwd_dq(const g4_problem* p, const void* q, g4_layout ql, const void*
   a.lse = lse;
   a.dq = (__bf16*)dq;
   a.dql = dql;
+  a.dq_list_clear = after_delta;
   hipError_t e = g4::launch_bwd_dq(a, (hipStream_t)stream);
   if (e != hipSuccess) return hip_fail(e, "backward dQ");
   return G4_OK;
+}
+
+int g4_attn_bwd_dq(const g4_problem* p, const void* q, g4_layout ql, const void* k, g4_layout kl,
+                   const void* v, g4_layout vl, const void* dout, g4_layout dol, const float* lse,
+                   void* dq, g4_layout dql, void* ws, size_t ws_bytes, void* stream) {
+  return bwd_dq(p, q, ql, k, kl, v, vl, dout, dol, lse, dq, dql, ws, ws_bytes, false, stream);
 }
 
 int g4_attn_bwd(const g4_problem* p, const void* q, g4_layout ql, const void* k, g4_layout kl,
@@ -671,8 +679,7 @@ int g4_attn_bwd(const g4_problem* p, const void* q, g4_layout ql, const void* k,
   if (nstripes == 0) {
     G4_TRY(g4_attn_bwd_dkdv(p, q, ql, k, kl, v, vl, dout, dol, lse, dk, dkl, dv, dvl, ws,
                             ws_bytes, stream));
-    G4_TRY(g4_attn_bwd_dq(p, q, ql, k, kl, v, vl, dout, dol, lse, dq, dql, ws, ws_bytes, stream));
-    return G4_OK;
+    return bwd_dq(p, q, ql, k, kl, v, vl, dout, dol, lse, dq, dql, ws, ws_bytes, true, stream);
   }
   // Striped stored dS (g4::for_each_ds_stripe): per stripe, the dK/dV launch
   // (which stores the stripe's dS; row stripes add to the fp32 dK / dV sums)

@@ -2197,7 +2197,7 @@ hipError_t launch_bwd_dq(const BwdParams& a, hipStream_t stream) {
   }
   if (a.p.head_dim == 256) {
     if (a.ds == nullptr) return launch_dq_roles_d<256>(a, stream);
-    if (a.dq_list != nullptr) {
+    if (a.dq_list != nullptr && !a.dq_list_clear) {
       // The list is refilled by every stored-dS pass (a fill kernel, not a
       // memset node, so the launch sequence can be captured in a graph).
       hipLaunchKernelGGL(clear_counter_kernel, dim3(1), dim3(64), 0, stream, a.sched + 3);

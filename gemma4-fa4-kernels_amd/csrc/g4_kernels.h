@@ -117,6 +117,9 @@ struct BwdParams {
   // for recomputation, appended by that pass ({sequence, query tile, query
   // head, 0}; order not significant: each entry writes its own dQ rows).
   int4* dq_list;
+  // The delta pass of this very call has just cleared the list's counter (the
+  // dQ stage on its own clears it first).
+  bool dq_list_clear;
 };
 
 // Workspace layout helpers (bytes).

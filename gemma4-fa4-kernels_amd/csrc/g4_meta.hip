@@ -98,53 +98,59 @@ __global__ void span_init_kernel(SpanWs w, int64_t nslots) {
   }
 }
 
+__device__ inline void span_insert_token(const g4_problem& p, SpanWs w, int64_t t) {
+  int vid = p.vision_ids[t];
+  if (vid < 0) return;
+  int s, lk;
+  int64_t ks;
+  seq_of_token(p, t, s, ks, lk);
+  // Only the ends of each run of equal keys (vision ID and document): a
+  // run's first position bounds its key's span from below and its last from
+  // above, so the other tokens add nothing (and every token of a block
+  // updating the same two words serialises on them: config 3's table took
+  // 24 us).
+  const unsigned long long key = span_key(p, t, vid);
+  const bool starts = t == ks || span_key(p, t - 1, p.vision_ids[t - 1]) != key;
+  const bool ends = t + 1 == ks + lk || span_key(p, t + 1, p.vision_ids[t + 1]) != key;
+  if (!starts && !ends) return;
+  int64_t slot = probe_slot(w, 2 * ks, 2 * (int64_t)lk, key, true);
+  if (slot < 0) return;
+  int j = (int)(t - ks);
+  if (starts) atomicMin(w.first + slot, j);
+  if (ends) atomicMax(w.last + slot, j);
+}
+
 __global__ void span_insert_kernel(g4_problem p, SpanWs w, int64_t tk) {
   for (int64_t t = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; t < tk;
-       t += (int64_t)gridDim.x * blockDim.x) {
-    int vid = p.vision_ids[t];
-    if (vid < 0) continue;
-    int s, lk;
-    int64_t ks;
-    seq_of_token(p, t, s, ks, lk);
-    // Only the ends of each run of equal keys (vision ID and document): a
-    // run's first position bounds its key's span from below and its last from
-    // above, so the other tokens add nothing (and every token of a block
-    // updating the same two words serialises on them: config 3's table took
-    // 24 us).
+       t += (int64_t)gridDim.x * blockDim.x)
+    span_insert_token(p, w, t);
+}
+
+__device__ inline void span_lookup_token(const g4_problem& p, SpanWs w, int64_t t) {
+  int s, lk;
+  int64_t ks;
+  seq_of_token(p, t, s, ks, lk);
+  int j = (int)(t - ks);
+  int vid = p.vision_ids[t];
+  int lo = j, hi = j;
+  if (vid >= 0) {
     const unsigned long long key = span_key(p, t, vid);
-    const bool starts = t == ks || span_key(p, t - 1, p.vision_ids[t - 1]) != key;
-    const bool ends = t + 1 == ks + lk || span_key(p, t + 1, p.vision_ids[t + 1]) != key;
-    if (!starts && !ends) continue;
-    int64_t slot = probe_slot(w, 2 * ks, 2 * (int64_t)lk, key, true);
-    if (slot < 0) continue;
-    int j = (int)(t - ks);
-    if (starts) atomicMin(w.first + slot, j);
-    if (ends) atomicMax(w.last + slot, j);
+    int64_t slot = probe_slot(w, 2 * ks, 2 * (int64_t)lk, key, false);
+    if (slot >= 0) {
+      lo = w.first[slot];
+      hi = w.last[slot];
+      // A run that starts after its key's first position: the key repeats.
+      if (lo < j && span_key(p, t - 1, p.vision_ids[t - 1]) != key) atomicOr(w.repeats, 1);
+    }
   }
+  w.lo[t] = lo;
+  w.hi[t] = hi;
 }
 
 __global__ void span_lookup_kernel(g4_problem p, SpanWs w, int64_t tk) {
   for (int64_t t = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; t < tk;
-       t += (int64_t)gridDim.x * blockDim.x) {
-    int s, lk;
-    int64_t ks;
-    seq_of_token(p, t, s, ks, lk);
-    int j = (int)(t - ks);
-    int vid = p.vision_ids[t];
-    int lo = j, hi = j;
-    if (vid >= 0) {
-      const unsigned long long key = span_key(p, t, vid);
-      int64_t slot = probe_slot(w, 2 * ks, 2 * (int64_t)lk, key, false);
-      if (slot >= 0) {
-        lo = w.first[slot];
-        hi = w.last[slot];
-        // A run that starts after its key's first position: the key repeats.
-        if (lo < j && span_key(p, t - 1, p.vision_ids[t - 1]) != key) atomicOr(w.repeats, 1);
-      }
-    }
-    w.lo[t] = lo;
-    w.hi[t] = hi;
-  }
+       t += (int64_t)gridDim.x * blockDim.x)
+    span_lookup_token(p, w, t);
 }
 
 // span_lo[j] = min{a >= off : M(a) >= j}, with M(a) the largest span end of
@@ -238,30 +244,114 @@ __global__ void __launch_bounds__(kReachChunk) span_chunk_scan_kernel(g4_problem
   }
 }
 
+// span_lo of token t from the prefix maxima m of its sequence (see above).
+__device__ inline int reach_token(const g4_problem& p, const int* first, int64_t t) {
+  int s, lk;
+  int64_t ks;
+  seq_of_token(p, t, s, ks, lk);
+  const Seq sq = resolve_seq(p, s);
+  if (sq.lq <= 0) return 0x7fffffff;  // no query attends this sequence's keys
+  const int j = (int)(t - ks);
+  const int* m = first + ks;
+  int l = max(lk - sq.lq, 0), r = lk - 1;  // the first a in [off, Sk) with M(a) >= j
+  while (l < r) {
+    const int mid = (l + r) >> 1;
+    if (m[mid] >= j)
+      r = mid;
+    else
+      l = mid + 1;
+  }
+  return l;
+}
+
 __global__ void span_reach_kernel(g4_problem p, SpanWs w, int64_t tk) {
   if (*w.repeats == 0) return;  // span_lo keeps the span starts
   for (int64_t t = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; t < tk;
-       t += (int64_t)gridDim.x * blockDim.x) {
+       t += (int64_t)gridDim.x * blockDim.x)
+    w.lo[t] = reach_token(p, w.first, t);
+}
+
+// All of the above in one workgroup, the hash table and the spans in LDS: up
+// to kSmallTokens K tokens and kSmallSeqs sequences.  At these sizes the passes
+// are their launches (a multimodal sample of 777 tokens: three in the forward,
+// six in the backward, 2-5 us each); one workgroup takes the same table and
+// the same passes, a workgroup barrier between them.
+constexpr int kSmallTokens = 4096;
+constexpr int kSmallSeqs = 256;
+constexpr int kSmallLds =
+    2 * kSmallTokens * 16 + (2 * (kSmallSeqs + 1) + kReachChunk / 64 + 1) * 4;
+static_assert(kSmallLds <= 160 * 1024, "LDS budget");
+
+__global__ void __launch_bounds__(kReachChunk) span_small_kernel(g4_problem p, SpanWs out, int tk,
+                                                                 bool query_reach) {
+  extern __shared__ __attribute__((aligned(16))) char smem_raw[];
+  constexpr int kPer = kSmallTokens / kReachChunk;
+  unsigned long long* keys = (unsigned long long*)smem_raw;
+  int* first = (int*)(keys + 2 * kSmallTokens);
+  int* last = first + 2 * kSmallTokens;
+  int* cu_q = last + 2 * kSmallTokens;
+  int* cu_k = cu_q + kSmallSeqs + 1;
+  int* wave_top = cu_k + kSmallSeqs + 1;
+  int* repeats = wave_top + kReachChunk / 64;
+  const int tid = threadIdx.x;
+  for (int i = tid; i < 2 * tk; i += kReachChunk) {
+    keys[i] = kEmpty;
+    first[i] = 0x7fffffff;
+    last[i] = -1;
+  }
+  if (tid == 0) *repeats = 0;
+  if (p.cu_seqlens_k != nullptr) {
+    if (tid <= p.num_seqs) {
+      cu_q[tid] = p.cu_seqlens_q[tid];
+      cu_k[tid] = p.cu_seqlens_k[tid];
+    }
+    p.cu_seqlens_q = cu_q;
+    p.cu_seqlens_k = cu_k;
+  }
+  __syncthreads();
+  SpanWs w = out;
+  w.keys = keys;
+  w.first = first;
+  w.last = last;
+  w.repeats = repeats;
+  for (int t = tid; t < tk; t += kReachChunk) span_insert_token(p, w, t);
+  __syncthreads();
+  // Thread's tokens: kPer adjacent ones (the scan below needs their order).
+  for (int i = 0; i < kPer; ++i)
+    if (tid * kPer + i < tk) span_lookup_token(p, w, tid * kPer + i);
+  __syncthreads();
+  if (!query_reach || *repeats == 0) return;
+  // M: the prefix maximum of ks + span_hi over query positions (chunk scan's).
+  long long m[kPer], top = -1;
+#pragma unroll
+  for (int i = 0; i < kPer; ++i) {
+    top = max(top, reach_end(p, w, (int64_t)tid * kPer + i, tk));  // (this thread's own hi)
+    m[i] = top;
+  }
+  const int lane = tid & 63, wv = tid >> 6;
+  long long v = top;
+#pragma unroll
+  for (int o = 1; o < 64; o <<= 1) {
+    const long long u = __shfl_up(v, o, 64);
+    if (lane >= o) v = max(v, u);
+  }
+  if (lane == 63) wave_top[wv] = (int)v;  // below 2^31: tk + tk at most
+  long long before = __shfl_up(v, 1, 64);
+  if (lane == 0) before = -1;
+  __syncthreads();
+  for (int x = 0; x < wv; ++x) before = max(before, (long long)wave_top[x]);
+#pragma unroll
+  for (int i = 0; i < kPer; ++i) {
+    const int t = tid * kPer + i;
+    if (t >= tk) break;
     int s, lk;
     int64_t ks;
     seq_of_token(p, t, s, ks, lk);
-    const Seq sq = resolve_seq(p, s);
-    if (sq.lq <= 0) {
-      w.lo[t] = 0x7fffffff;  // no query attends this sequence's keys
-      continue;
-    }
-    const int j = (int)(t - ks);
-    const int* m = w.first + ks;
-    int l = max(lk - sq.lq, 0), r = lk - 1;  // the first a in [off, Sk) with M(a) >= j
-    while (l < r) {
-      const int mid = (l + r) >> 1;
-      if (m[mid] >= j)
-        r = mid;
-      else
-        l = mid + 1;
-    }
-    w.lo[t] = l;
+    const long long g = max(before, m[i]);
+    first[t] = g >= ks ? (int)(g - ks) : -1;
   }
+  __syncthreads();
+  for (int t = tid; t < tk; t += kReachChunk) out.lo[t] = reach_token(p, first, t);
 }
 
 __global__ void mask_kernel(g4_problem p, uint8_t* out) {
@@ -346,6 +436,13 @@ size_t spans_bytes(const g4_problem& p) {
 hipError_t launch_spans(const g4_problem& p, void* ws, hipStream_t stream, bool query_reach) {
   int64_t tk = k_stream_tokens(p);
   SpanWs w = span_ws(ws, tk);
+  if (tk > 0 && tk <= kSmallTokens && p.num_seqs <= kSmallSeqs) {
+    static LdsAttr attr;
+    const hipError_t e = attr.ensure((const void*)span_small_kernel, kSmallLds);
+    if (e != hipSuccess) return e;
+    span_small_kernel<<<1, kReachChunk, kSmallLds, stream>>>(p, w, (int)tk, query_reach);
+    return hipGetLastError();
+  }
   span_init_kernel<<<grid_for(2 * tk, 256), 256, 0, stream>>>(w, 2 * tk);
   span_insert_kernel<<<grid_for(tk, 256), 256, 0, stream>>>(p, w, tk);
   span_lookup_kernel<<<grid_for(tk, 256), 256, 0, stream>>>(p, w, tk);
