@@ -72,13 +72,14 @@ def _check(source, weight, cos, sin) -> None:
         raise UnsupportedMI355XPath("the MI355X K/V preparation needs GPU tensors")
     if source.shape[-1] != _HEAD_DIM:
         raise UnsupportedMI355XPath("the MI355X K/V preparation covers head_dim 512")
-    if source.stride(-1) != 1 or any(s % 8 for s in source.stride()[:-1]) or \
-            source.data_ptr() % 16:
+    sb, sh, st, sd = source.stride()
+    if sd != 1 or sb % 8 or sh % 8 or st % 8 or source.data_ptr() % 16:
         raise ValueError("source needs a unit last-dim stride, outer strides that are "
                          "multiples of 8 and a 16-byte aligned base")
     if weight.shape != (source.shape[-1],):
         raise ValueError("k_norm_weight must have shape (head_dim,)")
-    if any(t.device != source.device for t in (weight, cos, sin)):
+    device = source.device
+    if weight.device != device or cos.device != device or sin.device != device:
         raise ValueError("source, k_norm_weight, cos and sin must share a device")
     if cos.requires_grad or sin.requires_grad:
         raise UnsupportedMI355XPath("gradients of cos / sin are not produced")
@@ -88,10 +89,6 @@ def _problem(source, rot, eps, stride, k_fp32) -> G4KvPrep:
     b, h, s, d = source.shape
     return G4KvPrep(num_batches=b, seqlen=s, num_heads=h, head_dim=d, rotary_dim=rot,
                     k_fp32=1 if k_fp32 else 0, eps=float(eps), cs_batch_stride=stride)
-
-
-def _stream(device):
-    return torch.cuda.current_stream(device).cuda_stream
 
 
 class _KvPrepFunction(torch.autograd.Function):
@@ -104,11 +101,12 @@ class _KvPrepFunction(torch.autograd.Function):
         prob = _problem(source, rot, eps, stride, k_fp32)
         k = torch.empty(source.shape, dtype=k_dtype, device=source.device)
         v = torch.empty(source.shape, dtype=source.dtype, device=source.device)
-        with torch.cuda.device(source.device):
+        out_layout = _layout(v)  # K's too: both contiguous, of the source's shape
+        with _lib.device_scope(source.device):
             _lib.check(lib.g4_kv_prep_fwd(
                 ctypes.byref(prob), source.data_ptr(), _layout(source), w.data_ptr(),
-                c.data_ptr(), s.data_ptr(), k.data_ptr(), _layout(k), v.data_ptr(),
-                _layout(v), _stream(source.device)))
+                c.data_ptr(), s.data_ptr(), k.data_ptr(), out_layout, v.data_ptr(),
+                out_layout, _lib.raw_stream(source.device)))
         ctx.save_for_backward(source, w, c, s)
         ctx.prob = prob
         ctx.weight_dtype = weight.dtype
@@ -127,16 +125,17 @@ class _KvPrepFunction(torch.autograd.Function):
         dk = dk.to(ctx.k_dtype).contiguous()
         dv = dv.to(source.dtype).contiguous()
         dz = torch.empty_like(source, memory_format=torch.contiguous_format)
+        grad_layout = _layout(dz)  # all three contiguous, of the source's shape
         dw = torch.empty(source.shape[-1], dtype=torch.float32, device=source.device)
         prob = ctx.prob
         ws = torch.empty(max(lib.g4_kv_prep_workspace_bytes(ctypes.byref(prob)), 16),
                          dtype=torch.uint8, device=source.device)
-        with torch.cuda.device(source.device):
+        with _lib.device_scope(source.device):
             _lib.check(lib.g4_kv_prep_bwd(
                 ctypes.byref(prob), source.data_ptr(), _layout(source), w.data_ptr(),
-                c.data_ptr(), s.data_ptr(), dk.data_ptr(), _layout(dk), dv.data_ptr(),
-                _layout(dv), dz.data_ptr(), _layout(dz), dw.data_ptr(), ws.data_ptr(), ws.numel(),
-                _stream(source.device)))
+                c.data_ptr(), s.data_ptr(), dk.data_ptr(), grad_layout, dv.data_ptr(),
+                grad_layout, dz.data_ptr(), grad_layout, dw.data_ptr(), ws.data_ptr(), ws.numel(),
+                _lib.raw_stream(source.device)))
         return dz, dw.to(ctx.weight_dtype), None, None, None, None, None
 
 
@@ -221,10 +220,10 @@ def prepare_rows_into(
     lib = _lib.load()
     prob = _problem(source, rotary_dim, eps, stride, k_fp32)
     null = G4Layout(0, 0, 0)
-    with torch.cuda.device(source.device):
+    with _lib.device_scope(source.device):
         _lib.check(lib.g4_kv_prep_fwd(
             ctypes.byref(prob), source.data_ptr(), _layout(source), w.data_ptr(),
             c.data_ptr() if c is not None else None, sn.data_ptr() if sn is not None else None,
             k.data_ptr() if k is not None else None, _layout(k) if k is not None else null,
             v.data_ptr() if v is not None else None, _layout(v) if v is not None else null,
-            _stream(source.device)))
+            _lib.raw_stream(source.device)))
