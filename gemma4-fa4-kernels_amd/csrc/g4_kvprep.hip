@@ -11,10 +11,10 @@
 //        dims pass through.  K in fp32 (fp32 tables): fp32 products and sum,
 //        no contraction.  K in bf16 (bf16 tables): each product and the sum
 //        rounded to bf16, as bf16 tensor operations round them.
-// One wave per row, lane l holding dims E l .. E l + E - 1 (E = D / 64: one
-// 16- or 8-byte load), so the row reduction is a wave reduction and rot(x) is
-// a lane exchange with lane l +- R / (2 E).  HBM-bound: each row reads 2 D
-// bytes of z and writes K and V (either may be left out).
+// Lane l of a row holds dims 8 l .. 8 l + 7 (one 16-byte load), so the row
+// reduction is a lane reduction and rot(x) an exchange with lane l +- R / 16.
+// HBM-bound: each row reads 2 D bytes of z and writes K and V (either may be
+// left out).
 //
 // Backward (D = 512; fp32 throughout, dz rounded to bf16 once):
 //   g_k  = adjoint of the RoPE applied to dK: i < R/2: dK_i cos_i + dK_{i+R/2} sin_{i+R/2};
@@ -41,19 +41,79 @@ __device__ __forceinline__ float wave_sum(float x) {
   return x;
 }
 
+// Rows enumerate (batch, token, head) with the head fastest.  64-bit divisions
+// and products were half of the forward's instructions, so below 2^31 rows and
+// with strides below 2^32 elements the row index is split with multipliers from
+// the host and an offset is three 32 x 32 + 64 bit multiply-adds (NARROW);
+// anything larger keeps the 64-bit form, and so does the backward, where it
+// made no difference (32.3 us for 32768 rows of 512 either way).
+struct RowMap {
+  uint32_t heads_mul, seq_mul;
+  int heads_shift, seq_shift;
+  bool narrow;
+};
+
+// n / d for n < 2^31 is (n * mul) >> (31 + shift), shift = ceil(log2 d),
+// mul = floor(2^(31 + shift) / d) + 1: the multiplier is too large by less than
+// one part in 2^31 / n, so the quotient is exact (Granlund and Montgomery).
+void division(uint32_t d, uint32_t& mul, int& shift) {
+  shift = 0;
+  while ((uint64_t(1) << shift) < d) ++shift;
+  mul = (uint32_t)((uint64_t(1) << (31 + shift)) / d + 1);
+}
+
+bool narrow_layout(const g4_layout& l) {
+  return ((l.batch_stride | l.token_stride | l.head_stride) >> 32) == 0;
+}
+
+template <class... L>
+RowMap row_map(const g4_kv_prep& p, const L&... layouts) {
+  RowMap m{};
+  const int64_t rows = (int64_t)p.num_batches * p.seqlen * p.num_heads;
+  m.narrow = rows < (int64_t(1) << 31) && (p.cs_batch_stride >> 32) == 0 &&
+             (narrow_layout(layouts) && ...);
+  if (m.narrow) {
+    division((uint32_t)p.num_heads, m.heads_mul, m.heads_shift);
+    division((uint32_t)p.seqlen, m.seq_mul, m.seq_shift);
+  }
+  return m;
+}
+
 struct RowAddr {
   int64_t b, t, h;
 };
 
 __device__ __forceinline__ RowAddr row_of(const g4_kv_prep& p, int64_t row) {
-  // rows enumerate (batch, token, head) with the head fastest
-  const int64_t h = row % p.num_heads;
   const int64_t bt = row / p.num_heads;
-  return RowAddr{bt / p.seqlen, bt % p.seqlen, h};
+  return RowAddr{bt / p.seqlen, bt % p.seqlen, row % p.num_heads};
 }
 
+template <bool NARROW>
+__device__ __forceinline__ RowAddr row_of(const g4_kv_prep& p, const RowMap& m, int64_t row) {
+  if constexpr (NARROW) {
+    const uint32_t n = (uint32_t)row;
+    const uint32_t bt = (uint32_t)(((uint64_t)n * m.heads_mul) >> (31 + m.heads_shift));
+    const uint32_t b = (uint32_t)(((uint64_t)bt * m.seq_mul) >> (31 + m.seq_shift));
+    return RowAddr{b, bt - b * (uint32_t)p.seqlen, n - bt * (uint32_t)p.num_heads};
+  }
+  return row_of(p, row);
+}
+
+template <bool NARROW>
+__device__ __forceinline__ int64_t product(int64_t i, int64_t stride) {
+  return NARROW ? (int64_t)((uint64_t)(uint32_t)i * (uint32_t)stride) : i * stride;
+}
+
+template <bool NARROW = false>
 __device__ __forceinline__ int64_t elem_off(const g4_layout& l, const RowAddr& a) {
-  return a.b * l.batch_stride + a.t * l.token_stride + a.h * l.head_stride;
+  return product<NARROW>(a.b, l.batch_stride) + product<NARROW>(a.t, l.token_stride) +
+         product<NARROW>(a.h, l.head_stride);
+}
+
+// Offset of a row's token in the cos / sin tables.
+template <bool NARROW>
+__device__ __forceinline__ int64_t table_off(const g4_kv_prep& p, const RowAddr& a) {
+  return product<NARROW>(a.b, p.cs_batch_stride) + product<NARROW>(a.t, p.rotary_dim);
 }
 
 __device__ __forceinline__ void load8(const __bf16* p, float (&x)[8]) {
@@ -69,6 +129,110 @@ __device__ __forceinline__ void store8(__bf16* p, const float (&x)[8]) {
   *(bf16x8*)p = v;
 }
 
+__device__ __forceinline__ void load8(const float* p, float (&x)[8]) {
+  const f32x4 lo = *(const f32x4*)p;
+  const f32x4 hi = *(const f32x4*)(p + 4);
+#pragma unroll
+  for (int e = 0; e < 4; ++e) {
+    x[e] = lo[e];
+    x[4 + e] = hi[e];
+  }
+}
+
+// D / 8 lanes per row, 8 dims (one 16-byte load) per lane: a wave takes one row
+// of 512 or two of 256.  Bound by instructions issued per row before it is by
+// HBM, hence two rows of 256 per instruction, partners exchanged as bf16 pairs
+// and the cheap row addresses: 32000 rows of 256 (K with RoPE) 14.9 -> 10.7 us,
+// 16000 rows 9.2 -> 7.4, 32768 rows of 512 (K in fp32, and V) 30.9 -> 26.4, at
+// 5 TB/s.
+template <int D, bool NARROW>
+__global__ void __launch_bounds__(kPrepWaves * 64) kv_prep_fwd_kernel(
+    g4_kv_prep p, RowMap map, const __bf16* z, g4_layout zl, const float* w, const float* cosv,
+    const float* sinv, void* k, g4_layout kl, __bf16* v, g4_layout vl, int64_t rows) {
+  constexpr int LPR = D / 8;  // lanes per row
+  const int lane = threadIdx.x & (LPR - 1);
+  const int64_t first = (int64_t)blockIdx.x * (kPrepWaves * 64 / LPR) + threadIdx.x / LPR;
+  const int64_t step = (int64_t)gridDim.x * (kPrepWaves * 64 / LPR);
+  const int rl = p.rotary_dim / 8;  // lanes holding rotary dims
+  const int half = rl / 2;          // lane distance of the rotate-half partner
+  float wl[8];
+  load8(w + 8 * lane, wl);
+  for (int64_t row = first; row < rows; row += step) {
+    const RowAddr a = row_of<NARROW>(p, map, row);
+    float x[8], c[8], s[8];
+    load8(z + elem_off<NARROW>(zl, a) + 8 * lane, x);
+    if (k != nullptr && lane < rl) {  // issued with z, before the row reduction waits for it
+      const int64_t t = table_off<NARROW>(p, a) + 8 * lane;
+      load8(cosv + t, c);
+      load8(sinv + t, s);
+    }
+    // Row sum of the rounded squares.  At 256 the two halves of a lane's dims
+    // are summed over the lanes apart and added last: the order of 64 lanes
+    // with 4 dims each.
+    float ss = 0.f, ss_hi = 0.f;
+    {
+#pragma clang fp contract(off)
+#pragma unroll
+      for (int e = 0; e < 8; ++e) (D == 256 && e >= 4 ? ss_hi : ss) += x[e] * x[e];
+    }
+    if constexpr (D == 256) {
+#pragma unroll
+      for (int o = 16; o > 0; o >>= 1) {
+        ss += __shfl_xor(ss, o, 64);
+        ss_hi += __shfl_xor(ss_hi, o, 64);
+      }
+      ss += ss_hi;
+    } else {
+      ss = wave_sum(ss);
+    }
+    const float r = 1.f / __fsqrt_rn(ss / (float)D + p.eps);
+    float n[8];
+    bf16x8 kb;
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
+      n[e] = x[e] * r;
+      kb[e] = (__bf16)(n[e] * wl[e]);
+    }
+    if (v != nullptr) store8(v + elem_off<NARROW>(vl, a) + 8 * lane, n);
+    if (k == nullptr) continue;
+    // rotate-half partner values, two bf16 per exchange (every lane of the row takes part)
+    const int partner = lane < half ? lane + half : lane - half;
+    const i32x4 kw = __builtin_bit_cast(i32x4, kb);
+    i32x4 pw;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) pw[e] = __shfl(kw[e], partner, LPR);
+    const bf16x8 pb = __builtin_bit_cast(bf16x8, pw);
+    float kout[8];
+#pragma unroll
+    for (int e = 0; e < 8; ++e) kout[e] = (float)kb[e];
+    if (lane < rl) {
+      // x * cos + rotate_half(x) * sin as two products and a sum, no fused
+      // multiply-add; in bf16 each product is rounded before the sum (the
+      // products of bf16 values are exact in fp32, so one rounding each)
+#pragma clang fp contract(off)
+      const float sign = lane < half ? -1.f : 1.f;
+#pragma unroll
+      for (int e = 0; e < 8; ++e) {
+        float a0 = kout[e] * c[e];
+        float a1 = (sign * (float)pb[e]) * s[e];
+        if (!p.k_fp32) {
+          a0 = (float)(__bf16)a0;
+          a1 = (float)(__bf16)a1;
+        }
+        kout[e] = a0 + a1;
+      }
+    }
+    const int64_t off = elem_off<NARROW>(kl, a) + 8 * lane;
+    if (p.k_fp32) {
+      float* kp = (float*)k + off;
+      *(f32x4*)kp = f32x4{kout[0], kout[1], kout[2], kout[3]};
+      *(f32x4*)(kp + 4) = f32x4{kout[4], kout[5], kout[6], kout[7]};
+    } else {
+      store8((__bf16*)k + off, kout);
+    }
+  }
+}
+
 // cos / sin of a row's token for this lane's dims (lanes below R / 8 only).
 __device__ __forceinline__ void load_rope(const g4_kv_prep& p, const float* cs, const RowAddr& a,
                                           int lane, float (&x)[8]) {
@@ -79,108 +243,6 @@ __device__ __forceinline__ void load_rope(const g4_kv_prep& p, const float* cs, 
   for (int e = 0; e < 4; ++e) {
     x[e] = lo[e];
     x[4 + e] = hi[e];
-  }
-}
-
-template <int E>
-using bf16v = __bf16 __attribute__((ext_vector_type(E)));
-
-// E consecutive bf16 / fp32 elements of this lane.
-template <int E>
-__device__ __forceinline__ void load_e(const __bf16* p, float (&x)[E]) {
-  const bf16v<E> v = *(const bf16v<E>*)p;
-#pragma unroll
-  for (int e = 0; e < E; ++e) x[e] = (float)v[e];
-}
-
-template <int E>
-__device__ __forceinline__ void store_e(__bf16* p, const float (&x)[E]) {
-  bf16v<E> v;
-#pragma unroll
-  for (int e = 0; e < E; ++e) v[e] = (__bf16)x[e];
-  *(bf16v<E>*)p = v;
-}
-
-template <int E>
-__device__ __forceinline__ void load_e(const float* p, float (&x)[E]) {
-#pragma unroll
-  for (int j = 0; j < E / 4; ++j) {
-    const f32x4 v = *(const f32x4*)(p + 4 * j);
-#pragma unroll
-    for (int e = 0; e < 4; ++e) x[4 * j + e] = v[e];
-  }
-}
-
-template <int E>
-__global__ void __launch_bounds__(kPrepWaves * 64) kv_prep_fwd_kernel(
-    g4_kv_prep p, const __bf16* z, g4_layout zl, const float* w, const float* cosv,
-    const float* sinv, void* k, g4_layout kl, __bf16* v, g4_layout vl, int64_t rows) {
-  constexpr int D = 64 * E;
-  const int lane = threadIdx.x & 63;
-  const int64_t first = (int64_t)blockIdx.x * kPrepWaves + (threadIdx.x >> 6);
-  const int64_t step = (int64_t)gridDim.x * kPrepWaves;
-  const int rl = p.rotary_dim / E;  // lanes holding rotary dims
-  const int half = rl / 2;          // lane distance of the rotate-half partner
-  float wl[E];
-  load_e<E>(w + E * lane, wl);
-  for (int64_t row = first; row < rows; row += step) {
-    const RowAddr a = row_of(p, row);
-    float x[E], c[E], s[E];
-    load_e<E>(z + elem_off(zl, a) + E * lane, x);
-    if (k != nullptr && lane < rl) {  // issued with z, before the row reduction waits for it
-      const int64_t t = a.b * p.cs_batch_stride + a.t * (int64_t)p.rotary_dim + E * lane;
-      load_e<E>(cosv + t, c);
-      load_e<E>(sinv + t, s);
-    }
-    float ss = 0.f;
-    {
-#pragma clang fp contract(off)
-#pragma unroll
-      for (int e = 0; e < E; ++e) ss += x[e] * x[e];  // rounded squares, then sums
-    }
-    ss = wave_sum(ss);
-    const float r = 1.f / __fsqrt_rn(ss / (float)D + p.eps);
-    float n[E], kn[E];
-#pragma unroll
-    for (int e = 0; e < E; ++e) {
-      n[e] = x[e] * r;
-      kn[e] = (float)(__bf16)(n[e] * wl[e]);
-    }
-    if (v != nullptr) store_e<E>(v + elem_off(vl, a) + E * lane, n);
-    if (k == nullptr) continue;
-    // rotate-half partner values (every lane takes part in the exchange)
-    const int partner = lane < half ? lane + half : lane - half;
-    float pk[E];
-#pragma unroll
-    for (int e = 0; e < E; ++e) pk[e] = __shfl(kn[e], partner, 64);
-    float kout[E];
-#pragma unroll
-    for (int e = 0; e < E; ++e) kout[e] = kn[e];
-    if (lane < rl) {
-      // x * cos + rotate_half(x) * sin as two products and a sum, no fused
-      // multiply-add; in bf16 each product is rounded before the sum (the
-      // products of bf16 values are exact in fp32, so one rounding each)
-#pragma clang fp contract(off)
-      const float sign = lane < half ? -1.f : 1.f;
-#pragma unroll
-      for (int e = 0; e < E; ++e) {
-        float a0 = kn[e] * c[e];
-        float a1 = (sign * pk[e]) * s[e];
-        if (!p.k_fp32) {
-          a0 = (float)(__bf16)a0;
-          a1 = (float)(__bf16)a1;
-        }
-        kout[e] = a0 + a1;
-      }
-    }
-    if (p.k_fp32) {
-      float* kp = (float*)k + elem_off(kl, a) + E * lane;
-#pragma unroll
-      for (int j = 0; j < E / 4; ++j)
-        *(f32x4*)(kp + 4 * j) = f32x4{kout[4 * j], kout[4 * j + 1], kout[4 * j + 2], kout[4 * j + 3]};
-    } else {
-      store_e<E>((__bf16*)k + elem_off(kl, a) + E * lane, kout);
-    }
   }
 }
 
@@ -320,15 +382,14 @@ hipError_t launch_kv_prep_fwd(const g4_kv_prep& p, const void* z, g4_layout zl, 
                               void* v, g4_layout vl, hipStream_t stream) {
   const int64_t rows = (int64_t)p.num_batches * p.seqlen * p.num_heads;
   if (rows <= 0) return hipSuccess;
-  const int fwd_blocks = (int)std::min<int64_t>((rows + kPrepWaves - 1) / kPrepWaves, 4096);
-  if (p.head_dim == 256)
-    hipLaunchKernelGGL(kv_prep_fwd_kernel<4>, dim3(fwd_blocks), dim3(kPrepWaves * 64), 0,
-                       stream, p, (const __bf16*)z, zl, w, cosv, sinv, k, kl, (__bf16*)v, vl,
-                       rows);
-  else
-    hipLaunchKernelGGL(kv_prep_fwd_kernel<8>, dim3(fwd_blocks), dim3(kPrepWaves * 64), 0,
-                       stream, p, (const __bf16*)z, zl, w, cosv, sinv, k, kl, (__bf16*)v, vl,
-                       rows);
+  const int per_block = kPrepWaves * 512 / p.head_dim;
+  const int blocks = (int)std::min<int64_t>((rows + per_block - 1) / per_block, 4096);
+  const RowMap map = row_map(p, zl, k != nullptr ? kl : zl, v != nullptr ? vl : zl);
+  const auto kernel = p.head_dim == 256
+                          ? (map.narrow ? kv_prep_fwd_kernel<256, true> : kv_prep_fwd_kernel<256, false>)
+                          : (map.narrow ? kv_prep_fwd_kernel<512, true> : kv_prep_fwd_kernel<512, false>);
+  hipLaunchKernelGGL(kernel, dim3(blocks), dim3(kPrepWaves * 64), 0, stream, p, map,
+                     (const __bf16*)z, zl, w, cosv, sinv, k, kl, (__bf16*)v, vl, rows);
   return hipGetLastError();
 }
 
