@@ -57,7 +57,8 @@ __device__ __forceinline__ void issue_meta(const g4_problem& p, const Seq& sq, i
 constexpr float kRescaleLog2 = 8.0f;
 
 // META: key metadata kinds compiled in (bit 0 vision IDs, bit 1 document IDs).
-template <int D, int BN, int DSPLIT, int NQG, bool VDOUBLE, int META, int OCC = 1>
+// KS: wave groups that share the key tiles, each taking every KS-th one.
+template <int D, int BN, int DSPLIT, int NQG, bool VDOUBLE, int META, int OCC = 1, int KS = 1>
 struct FwdKernel {
   using C = FwdCfg<D, BN, DSPLIT, NQG, VDOUBLE>;
   static constexpr int kNB = C::kDH / 32;  // 32-wide head-dim blocks per wave
@@ -77,7 +78,7 @@ struct FwdKernel {
   // Head dim 512 keeps the compiler's wait before the P.V reads: with it the
   // 8192-token causal forward measured 2.81 ms, without it 2.91 ms.
   TrReader<C::kCPR, (D != 512)> vrd;
-  TileCopier<C::kCPR, BN, C::kNW, (OCC > 1)> kcp, vcp;
+  TileCopier<C::kCPR, BN, C::kNW, (OCC * KS > 1)> kcp, vcp;
   bf16x8 qf[kNC];
   f32x16 o_acc[kNB];
   float m_run, l_run;
@@ -153,8 +154,8 @@ struct FwdKernel {
   // caller issues K(0), V(0) and K(1) first.
   template <bool AHEAD = false>
   __device__ __forceinline__ void step(int cur, int it, int ntiles, int t_first) {
-    static_assert(!AHEAD || (VDOUBLE && META == 0), "K-ahead steps");
-    const int kb0 = (t_first + it) * BN;
+    static_assert(!AHEAD || (VDOUBLE && META == 0 && KS == 1), "K-ahead steps");
+    const int kb0 = (t_first + it * KS) * BN;
     // This wave's copies of K (and, double-buffered, V) for this tile have
     // landed; the barrier publishes every wave's copies and ends all reads of
     // the buffers refilled below.  (AHEAD: K(it + 1), issued last, may still
@@ -173,9 +174,9 @@ struct FwdKernel {
     if constexpr (AHEAD) {
       if (it + 1 < ntiles) issue_v(kb0 + BN, cur ^ 1);
     } else if (it + 1 < ntiles) {
-      issue_k(kb0 + BN, cur ^ 1);
-      if (has_meta && wave == 0) issue_meta(*p, sq, kb0 + BN, smem + C::kLdsMeta + (cur ^ 1) * 512, lane, has_vid, has_doc);
-      if constexpr (VDOUBLE) issue_v(kb0 + BN, cur ^ 1);
+      issue_k(kb0 + KS * BN, cur ^ 1);
+      if (has_meta && wave == 0) issue_meta(*p, sq, kb0 + KS * BN, smem + C::kLdsMeta + (cur ^ 1) * 512, lane, has_vid, has_doc);
+      if constexpr (VDOUBLE) issue_v(kb0 + KS * BN, cur ^ 1);
     }
 
     // S^T partial over this wave's head-dim slice.
@@ -296,7 +297,7 @@ struct FwdKernel {
     if constexpr (!VDOUBLE) {
       // Single V buffer: every wave must finish its PV reads before refill.
       barrier_lds();
-      if (it + 1 < ntiles) issue_v(kb0 + BN, 0);
+      if (it + 1 < ntiles) issue_v(kb0 + KS * BN, 0);
     }
   }
 };
@@ -396,19 +397,93 @@ static int64_t fwd_grid(FwdParams* b, int bm, bool allow_compact) {
   return n;
 }
 
+// Two groups of waves of one workgroup with the same queries and every second
+// key tile each (KS = 2).
+template <class C>
+struct FwdKeyGroups {
+  static constexpr int kGroupLds = (C::kLdsBytes + 1023) / 1024 * 1024;
+  static constexpr int kNB = C::kDH / 32;
+  static constexpr int kHalf = kNB / 2 * 4096;               // half of a wave's accumulators
+  static constexpr int kLdsState = 2 * C::kNW * kHalf;       // [group][wave][m, l][lane] fp32
+  static constexpr int kLdsBytes = std::max(2 * kGroupLds, kLdsState + 2 * C::kNW * 512);
+  static_assert(kLdsBytes <= 160 * 1024, "LDS budget");
+
+  // Group G finishes half G of the head dim: it sends the other half of its
+  // accumulators, and its m and l, through LDS, and with M the larger m,
+  // O = sum 2^(m_g - M) O_g / sum 2^(m_g - M) l_g.
+  template <int G, class K>
+  __device__ static __forceinline__ void finish(const FwdParams& a, K& ker, char* smem_all, int s,
+                                                int qh, int my_i, bool q_valid) {
+    char G4_LDS* smem = (char G4_LDS*)smem_all;
+    const int lane = ker.lane, wave = ker.wave;
+    const float l_mine = ker.l_run + wave_xor32(ker.l_run);
+    barrier_lds();  // both groups are done with their tiles
+    char G4_LDS* send = smem + (G * C::kNW + wave) * kHalf + lane * 16;
+    const char G4_LDS* recv = smem + ((1 - G) * C::kNW + wave) * kHalf + lane * 16;
+    float G4_LDS* st = (float G4_LDS*)(smem + kLdsState);
+#pragma unroll
+    for (int b = 0; b < kNB / 2; ++b)
+#pragma unroll
+      for (int r4 = 0; r4 < 4; ++r4) {
+        const f32x16& x = ker.o_acc[(1 - G) * (kNB / 2) + b];
+        *(f32x4 G4_LDS*)(send + (b * 4 + r4) * 1024) =
+            f32x4{x[r4 * 4], x[r4 * 4 + 1], x[r4 * 4 + 2], x[r4 * 4 + 3]};
+      }
+    st[(G * C::kNW + wave) * 128 + lane] = ker.m_run;
+    st[(G * C::kNW + wave) * 128 + 64 + lane] = l_mine;
+    barrier_lds();
+    const float m_other = st[((1 - G) * C::kNW + wave) * 128 + lane];
+    const float l_other = st[((1 - G) * C::kNW + wave) * 128 + 64 + lane];
+    const float m = fmaxf(ker.m_run, m_other);
+    const float m_use = m == kNegInf ? 0.f : m;
+    const float f_mine = fast_exp2(ker.m_run - m_use), f_other = fast_exp2(m_other - m_use);
+    const float l_tot = l_mine * f_mine + l_other * f_other;
+    const float inv = l_tot > 0.f ? 1.f / l_tot : 0.f;
+    if (!q_valid) return;
+    __bf16* orow = a.o + tok_off(ker.sq, s, ker.sq.qtok, my_i, a.ol) +
+                   (int64_t)qh * a.ol.head_stride + G * (C::kDH / 2) + 4 * ker.h32;
+#pragma unroll
+    for (int b = 0; b < kNB / 2; ++b)
+#pragma unroll
+      for (int r4 = 0; r4 < 4; ++r4) {
+        const f32x16& x = ker.o_acc[G * (kNB / 2) + b];
+        const f32x4 y = *(const f32x4 G4_LDS*)(recv + (b * 4 + r4) * 1024);
+        bf16x4 v;
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+          v[e] = (__bf16)((x[r4 * 4 + e] * f_mine + y[e] * f_other) * inv);
+        *(bf16x4*)(orow + b * 32 + 8 * r4) = v;
+      }
+    if (G == 0 && ker.h32 == 0)
+      a.lse[lse_off(a.p, ker.sq, s, qh, my_i)] =
+          l_tot > 0.f ? (m + fast_log2(l_tot)) * kLn2 : kNegInf;
+  }
+};
+
 // One work item L of the forward (one query tile of one head).
 // FIXUP: item L of the rescaling pass (FixupItem).
 // OCC: workgroups per CU the register budget is sized for.
-template <int D, int BN, int DSPLIT, int NQG, bool VDOUBLE, int META, bool FIXUP, int OCC>
-__device__ __forceinline__ void fwd_item(const FwdParams& a, char* smem_raw, int L) {
-  using K = FwdKernel<D, BN, DSPLIT, NQG, VDOUBLE, META, OCC>;
+// KS = 2: two groups of waves, each with LDS of its own, take the even and the
+// odd key tiles; their states are combined at the end.
+template <int D, int BN, int DSPLIT, int NQG, bool VDOUBLE, int META, bool FIXUP, int OCC,
+          int KS = 1>
+__device__ __forceinline__ void fwd_item(const FwdParams& a, char* smem_all, int L) {
+  using K = FwdKernel<D, BN, DSPLIT, NQG, VDOUBLE, META, OCC, KS>;
   using C = typename K::C;
+  static_assert(KS == 1 || (KS == 2 && DSPLIT == 1 && VDOUBLE && !FIXUP && META != 3),
+                "key groups");
   K ker;
+  int kg = 0;  // this wave's group
+  char* smem_raw = smem_all;
+  if constexpr (KS > 1) {
+    kg = __builtin_amdgcn_readfirstlane(threadIdx.x / C::kNT);
+    smem_raw += kg * FwdKeyGroups<C>::kGroupLds;
+  }
   ker.smem = (char G4_LDS*)smem_raw;
   ker.p = &a.p;
   const g4_problem& p = a.p;
 
-  ker.tid = threadIdx.x;
+  ker.tid = KS > 1 ? threadIdx.x % C::kNT : threadIdx.x;
   ker.lane = ker.tid & 63;
   ker.wave = __builtin_amdgcn_readfirstlane(ker.tid >> 6);
   const int qg = ker.wave / DSPLIT;
@@ -462,8 +537,13 @@ __device__ __forceinline__ void fwd_item(const FwdParams& a, char* smem_raw, int
   }
   int klo, khi;
   query_tile_key_range(ker.a0, a_last_valid, sq.lk, p.window, span_max, klo, khi);
-  const int t_first = klo / BN;
-  const int ntiles = (khi + BN - 1) / BN - t_first;
+  int t_first = klo / BN;
+  int ntiles = (khi + BN - 1) / BN - t_first;
+  const int all_tiles = ntiles;
+  if constexpr (KS > 1) {  // this group's
+    t_first += kg;
+    ntiles = max((all_tiles - kg + KS - 1) / KS, 0);
+  }
   // ---- document uniformity -------------------------------------------------
   // The range spans whole 64-key tiles (a superset of the visited tiles for
   // BN <= 64), so both launches of a split problem evaluate it identically.
@@ -530,6 +610,15 @@ __device__ __forceinline__ void fwd_item(const FwdParams& a, char* smem_raw, int
   // (Two tiles per iteration with compile-time buffers measured slower: the
   // unrolled loop spills.)
   for (int it = 0; it < ntiles; ++it) ker.step(it & 1, it, ntiles, t_first);
+  if constexpr (KS > 1) {
+    // a step has one barrier; the second group may have a step less
+    if (kg > 0 && all_tiles > 0 && all_tiles % KS) barrier_lds();
+    if (kg == 0)
+      FwdKeyGroups<C>::template finish<0>(a, ker, smem_all, s, qh, my_i, q_valid);
+    else
+      FwdKeyGroups<C>::template finish<1>(a, ker, smem_all, s, qh, my_i, q_valid);
+    return;
+  }
 
   // ---- epilogue: normalise, write O and LSE ---------------------------------
   const float l_tot = ker.l_run + wave_xor32(ker.l_run);
@@ -555,8 +644,8 @@ __device__ __forceinline__ void fwd_item(const FwdParams& a, char* smem_raw, int
 }
 
 template <int D, int BN, int DSPLIT, int NQG, bool VDOUBLE, int META, bool FIXUP = false,
-          int OCC = 1>
-__global__ void __launch_bounds__(NQG * DSPLIT * 64, OCC) fwd_kernel(FwdParams a) {
+          int OCC = 1, int KS = 1>
+__global__ void __launch_bounds__(NQG * DSPLIT * KS * 64, OCC) fwd_kernel(FwdParams a) {
   using C = FwdCfg<D, BN, DSPLIT, NQG, VDOUBLE>;
   extern __shared__ __attribute__((aligned(16))) char smem_raw[];
   if constexpr (META == 3 && !FIXUP) {
@@ -592,7 +681,8 @@ __global__ void __launch_bounds__(NQG * DSPLIT * 64, OCC) fwd_kernel(FwdParams a
       }
     }
   } else {
-    fwd_item<D, BN, DSPLIT, NQG, VDOUBLE, META, FIXUP, OCC>(a, smem_raw, FwdItem::of_block(a));
+    fwd_item<D, BN, DSPLIT, NQG, VDOUBLE, META, FIXUP, OCC, KS>(a, smem_raw,
+                                                                FwdItem::of_block(a));
   }
 }
 
@@ -1798,6 +1888,36 @@ static hipError_t launch_fwd_cfg(const FwdParams& a, hipStream_t stream, bool fi
   return hipGetLastError();
 }
 
+constexpr int kCus = 256;
+
+// Two groups of waves per query tile (KS = 2, head dim 256): one workgroup of
+// 8 waves per CU in place of two of 4 waves.  With more tiles than CUs the two
+// workgroups fill a CU by themselves, and drift apart, so that one's softmax
+// meets the other's matrix steps; up to 256 tiles each would run alone on its
+// CU, bound by its own chain of steps (32 of 1.25 us at 1024 keys, 0.43 us of
+// them in the matrix cores).  Sharing the keys makes it 16 steps of 2.0 us and
+// 1.3 us for the exchange, which pays from about 256 keys on: 32 heads over
+// 1024 tokens 46.5 -> 38.6 us, 777 tokens 37.6 -> 31.9, 64 new tokens after
+// 1023 cached (4 sequences) 45.7 -> 35.9, 400 tokens 23.5 -> 22.1; at 256
+// 18.5 -> 18.3, at 128 13.6 -> 15.1.
+static bool use_fwd_groups(const g4_problem& p, int64_t nblocks) {
+  const int64_t keys =
+      p.window > 0 ? std::min<int64_t>(p.seqlen_k, (int64_t)p.window + 127) : p.seqlen_k;
+  return nblocks > 0 && nblocks <= kCus && keys > 256;
+}
+
+template <int META>
+static hipError_t launch_fwd_groups(const FwdParams& a, int64_t nblocks, hipStream_t stream) {
+  using C = FwdCfg<256, 32, 1, 4, true>;
+  const auto kern = fwd_kernel<256, 32, 1, 4, true, META, false, 1, 2>;
+  static LdsAttr attr;
+  hipError_t e = attr.ensure((const void*)kern, FwdKeyGroups<C>::kLdsBytes);
+  if (e != hipSuccess) return e;
+  hipLaunchKernelGGL(kern, dim3((unsigned)nblocks), dim3(2 * C::kNT), FwdKeyGroups<C>::kLdsBytes,
+                     stream, a);
+  return hipGetLastError();
+}
+
 __global__ void clear_list_kernel(unsigned* n) {
   if (threadIdx.x == 0) *n = 0u;
 }
@@ -1815,7 +1935,19 @@ hipError_t launch_fwd(const FwdParams& a, hipStream_t stream) {
     // one workgroup of 64-key tiles per CU, so such a problem is split: the
     // query tiles that see a single document run in the vision-only kernel,
     // the rest in the full-mask one.
-    if (meta_kind(a.p) != 3) return launch_fwd_cfg<256, 32, 1, 4, true, 2>(a, stream);
+    if (meta_kind(a.p) != 3) {
+      FwdParams b = a;
+      b.doc_pass = 0;
+      const int64_t n = fwd_grid(&b, FwdCfg<256, 32, 1, 4, true>::kBM, true);
+      if (use_fwd_groups(a.p, n)) {
+        switch (meta_kind(a.p)) {
+          case 1: return launch_fwd_groups<1>(b, n, stream);
+          case 2: return launch_fwd_groups<2>(b, n, stream);
+          default: return launch_fwd_groups<0>(b, n, stream);
+        }
+      }
+      return launch_fwd_cfg<256, 32, 1, 4, true, 2>(a, stream);
+    }
     static_assert(FwdCfg<256, 32, 1, 4, true>::kBM == FwdCfg<256, 64, 1, 4, true>::kBM,
                   "both passes must tile queries alike");
     if (a.doc_list_n != nullptr) {
