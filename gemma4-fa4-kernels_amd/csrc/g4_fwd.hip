@@ -345,30 +345,141 @@ struct FwdItem {
   }
 };
 
-// Item L of the rescaling pass after the wide kernel: 64 queries (tile qt) of
-// one head of sequence s, heads innermost.
+// Item of the rescaling pass after the wide kernel: 64 queries (tile qt) of one
+// head of sequence s.
 struct FixupItem {
   static constexpr int kBM = 64;
   int s, qt, qh;
-  __device__ __forceinline__ FixupItem(const FwdParams& a, int L) {
-    const int hq = a.p.num_q_heads;
-    qh = L % hq;
-    qt = L / hq % a.ntq;
-    s = L / hq / a.ntq;
+};
+
+// The rescaling pass's items, in the order of blocks of four tiles (a sequence's
+// last ones first; then sequence and KV head), their tiles from the last on and
+// the heads of a tile.  Flagged items are few and lie anywhere (one head, one row
+// of every head, one sequence), and each walks a whole key range, so no fixed
+// share of all items balances the workgroups: every workgroup reads the flags (4
+// bytes per 32 queries and head), and the flagged items are dealt in order,
+// forwards in the even rounds and backwards in the odd ones (a round's last item
+// costs least).  Neighbours (an XCD's 32 workgroups take 32 in a row) then walk the
+// same keys at the same time: 8192 tokens with every row flagged, tiles taken in
+// zigzag order instead 7.9 ms, one tile of all KV heads 5.6.
+struct FixupScan {
+  static constexpr int kTiles = 4;   // tiles of a block: one thread's in a step
+  static constexpr int kMine = 64;   // a step's items of one workgroup, at most
+  static constexpr int kLdsBytes = kMine * 16 + 64;
+  const FwdParams& a;
+  int grp;
+  int64_t segs, blocks;
+  __device__ __forceinline__ explicit FixupScan(const FwdParams& x) : a(x) {
+    grp = a.p.num_q_heads / a.p.num_kv_heads;
+    segs = (int64_t)a.num_seqs * a.p.num_kv_heads;
+    blocks = segs * ((a.ntq + kTiles - 1) / kTiles);
   }
-  // Whether the wide kernel flagged a row group of these queries and KV head
-  // (raise_flags; the group's heads share their slots).
-  __device__ __forceinline__ bool flagged(const FwdParams& a) const {
-    const g4_problem& p = a.p;
-    const int lq = p.cu_seqlens_q ? p.cu_seqlens_q[s + 1] - p.cu_seqlens_q[s] : p.seqlen_q;
-    const int grp = p.num_q_heads / p.num_kv_heads;
-    const int nq32 = (p.seqlen_q + 31) / 32;
-    int any = 0;
-    for (int q32 = qt * 2; q32 < qt * 2 + 2 && q32 * 32 < lq; ++q32) {
-      const int* f = a.raise_flags + ((int64_t)s * nq32 + q32) * p.num_q_heads + qh / grp * grp;
-      for (int j = 0; j < grp; ++j) any |= f[j];
+  // Block u: tiles t0 .. t0 + 3 of sequence s.
+  __device__ __forceinline__ void locate(int64_t u, int& s, int& t0, int& kvh) const {
+    const int hkv = a.p.num_kv_heads, nb = (a.ntq + kTiles - 1) / kTiles;
+    if (blocks < (int64_t(1) << 31)) {  // (32-bit divisions, a tenth of the 64-bit ones' cost)
+      const uint32_t t = (uint32_t)u / (uint32_t)segs, g = (uint32_t)u - t * (uint32_t)segs;
+      s = (int)(g / (uint32_t)hkv);
+      kvh = (int)(g - (uint32_t)s * (uint32_t)hkv);
+      t0 = (nb - 1 - (int)t) * kTiles;
+      return;
     }
-    return any != 0;
+    const int64_t t = u / segs, g = u - t * segs;
+    s = (int)(g / hkv);
+    kvh = (int)(g - (int64_t)s * hkv);
+    t0 = (nb - 1 - (int)t) * kTiles;
+  }
+  // Heads of a block's tiles with a row that the wide kernel could not finish, a
+  // bit each: 8 bits per tile, the last tile's lowest.  (GRP at compile time, so
+  // that the loads are in flight together.)
+  template <int GRP>
+  __device__ __forceinline__ unsigned heads(int64_t u) const {
+    if (u >= blocks) return 0;
+    int s, t0, kvh;
+    locate(u, s, t0, kvh);
+    const g4_problem& p = a.p;
+    const int nq32 = (p.seqlen_q + 31) / 32;
+    const int lq = p.cu_seqlens_q ? p.cu_seqlens_q[s + 1] - p.cu_seqlens_q[s] : p.seqlen_q;
+    const int* f = a.raise_flags + (int64_t)s * nq32 * p.num_q_heads + kvh * GRP;
+    constexpr int kVec = GRP < 4 ? GRP : 4;
+    typedef int vec __attribute__((ext_vector_type(kVec)));
+    vec x[2 * kTiles][GRP / kVec];
+#pragma unroll
+    for (int i = 0; i < 2 * kTiles; ++i)
+#pragma unroll
+      for (int j = 0; j < GRP / kVec; ++j)
+        x[i][j] = *(const vec*)(f + (int64_t)min(t0 * 2 + i, nq32 - 1) * p.num_q_heads + j * kVec);
+    unsigned any = 0;
+#pragma unroll
+    for (int i = 0; i < 2 * kTiles; ++i) {
+      int m = 0;
+#pragma unroll
+      for (int j = 0; j < GRP; ++j) m |= x[i][j / kVec][j % kVec];
+      // 32-query groups past the sequence's end hold nothing
+      any |= (t0 * 2 + i) * 32 < lq ? (unsigned)m << 8 * (kTiles - 1 - i / 2) : 0u;
+    }
+    return any;
+  }
+  __device__ __forceinline__ unsigned heads(int64_t u) const {
+    switch (grp) {
+      case 1: return heads<1>(u);
+      case 2: return heads<2>(u);
+      case 4: return heads<4>(u);
+      default: return heads<8>(u);
+    }
+  }
+  // Runs run(item) for every flagged item of this workgroup; all threads call
+  // it.  lds: kLdsBytes that run() leaves alone.
+  template <class Run>
+  __device__ __forceinline__ void each(char G4_LDS* lds, Run run) const {
+    i32x4 G4_LDS* list = (i32x4 G4_LDS*)lds;
+    int G4_LDS* wave_sum = (int G4_LDS*)(lds + kMine * 16);  // [step parity][wave]
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, nt = blockDim.x;
+    const int n = gridDim.x, me = xcd_remap(blockIdx.x, n);
+    auto number = [&](int64_t round) { return round * n + (round & 1 ? n - 1 - me : me); };
+    int64_t before = 0;  // flagged items of the earlier steps
+    int par = 0;
+    for (int64_t u0 = 0; u0 < blocks; u0 += nt, par ^= 1) {
+      const unsigned any = heads(u0 + tid);
+      const int cnt = __popc(any);
+      int incl = cnt;
+      if (__ballot(cnt != 0)) {
+#pragma unroll
+        for (int o = 1; o < 64; o <<= 1) {
+          const int y = __shfl_up(incl, o, 64);
+          if (lane >= o) incl += y;
+        }
+      }
+      if (lane == 63) wave_sum[par * 8 + wave] = incl;
+      barrier_lds();  // (and the previous step's list has been read)
+      int total = 0;
+      int64_t rank = before + incl - cnt;
+      for (int w = 0; w < nt / 64; ++w) {
+        const int x = wave_sum[par * 8 + w];
+        if (w < wave) rank += x;
+        total += x;
+      }
+      total = __builtin_amdgcn_readfirstlane(total);
+      if (total == 0) continue;
+      const int64_t round0 = before / n, end = before + total;
+      for (unsigned m = any; m; m &= m - 1, ++rank) {
+        const int64_t round = rank / n;
+        if (rank != number(round)) continue;
+        const int bit = __ffs(m) - 1;
+        int s, t0, kvh;
+        locate(u0 + tid, s, t0, kvh);
+        list[round - round0] = i32x4{s, t0 + kTiles - 1 - bit / 8, kvh * grp + bit % 8, 0};
+      }
+      barrier_lds();
+      for (int64_t round = round0; round * n < end; ++round) {
+        const int64_t r = number(round);
+        if (r < before || r >= end) continue;
+        const i32x4 it = list[round - round0];
+        run(FixupItem{__builtin_amdgcn_readfirstlane(it[0]), __builtin_amdgcn_readfirstlane(it[1]),
+                      __builtin_amdgcn_readfirstlane(it[2])});
+      }
+      before = end;
+    }
   }
 };
 
@@ -461,13 +572,14 @@ struct FwdKeyGroups {
 };
 
 // One work item L of the forward (one query tile of one head).
-// FIXUP: item L of the rescaling pass (FixupItem).
+// FIXUP: the item `fix` of the rescaling pass (L is not used).
 // OCC: workgroups per CU the register budget is sized for.
 // KS = 2: two groups of waves, each with LDS of its own, take the even and the
 // odd key tiles; their states are combined at the end.
 template <int D, int BN, int DSPLIT, int NQG, bool VDOUBLE, int META, bool FIXUP, int OCC,
           int KS = 1>
-__device__ __forceinline__ void fwd_item(const FwdParams& a, char* smem_all, int L) {
+__device__ __forceinline__ void fwd_item(const FwdParams& a, char* smem_all, int L,
+                                         FixupItem fix = {}) {
   using K = FwdKernel<D, BN, DSPLIT, NQG, VDOUBLE, META, OCC, KS>;
   using C = typename K::C;
   static_assert(KS == 1 || (KS == 2 && DSPLIT == 1 && VDOUBLE && !FIXUP && META != 3),
@@ -495,11 +607,10 @@ __device__ __forceinline__ void fwd_item(const FwdParams& a, char* smem_all, int
   FwdItem it;
   int kvh, qh, s, qt;
   if constexpr (FIXUP) {
-    const FixupItem f(a, L);
-    kvh = f.qh / (p.num_q_heads / p.num_kv_heads);
-    qh = f.qh;
-    s = f.s;
-    qt = f.qt;
+    kvh = fix.qh / (p.num_q_heads / p.num_kv_heads);
+    qh = fix.qh;
+    s = fix.s;
+    qt = fix.qt;
   } else {
     if (!it.decode(a, L, C::kBM)) return;
     kvh = it.kvh;
@@ -662,24 +773,14 @@ __global__ void __launch_bounds__(NQG * DSPLIT * KS * 64, OCC) fwd_kernel(FwdPar
       fwd_item<D, BN, DSPLIT, NQG, VDOUBLE, META, FIXUP, OCC>(a, smem_raw, L);
     }
   } else if constexpr (FIXUP) {
-    // Rescaling pass: items blockIdx.x, + gridDim.x, ... tested 64 at a time,
-    // one per lane (every wave the same), the flagged ones run.  Flags are
-    // rare, so the pass is its test: one workgroup per item spent 119 us on
-    // 33792 workgroups of 32 packed sequences (32768 tokens).
+    // Rescaling pass.  Flags are rare, so the pass is its reading of them: one
+    // workgroup per item spent 119 us on 33792 workgroups of 32 packed sequences
+    // (32768 tokens).
     static_assert(C::kBM == FixupItem::kBM, "rescaling tiles");
-    const int n = a.num_seqs * a.ntq * a.p.num_q_heads;
-    const int lane = threadIdx.x & 63;
-    for (int64_t base = blockIdx.x; base < n; base += (int64_t)64 * gridDim.x) {
-      const int64_t mine = base + (int64_t)lane * gridDim.x;
-      unsigned long long todo = __ballot(mine < n && FixupItem(a, (int)mine).flagged(a));
-      while (todo) {
-        const int b = __builtin_amdgcn_readfirstlane(__ffsll((long long)todo) - 1);
-        todo &= todo - 1;
-        barrier_lds();  // the previous item's LDS reads are done
-        fwd_item<D, BN, DSPLIT, NQG, VDOUBLE, META, FIXUP, OCC>(a, smem_raw,
-                                                                (int)(base + b * gridDim.x));
-      }
-    }
+    FixupScan(a).each((char G4_LDS*)smem_raw + C::kLdsBytes, [&](const FixupItem& it) {
+      barrier_lds();  // the previous item's LDS reads are done
+      fwd_item<D, BN, DSPLIT, NQG, VDOUBLE, META, FIXUP, OCC>(a, smem_raw, 0, it);
+    });
   } else {
     fwd_item<D, BN, DSPLIT, NQG, VDOUBLE, META, FIXUP, OCC, KS>(a, smem_raw,
                                                                 FwdItem::of_block(a));
@@ -1340,9 +1441,9 @@ static hipError_t launch_fwd_decode(const FwdParams& a, hipStream_t stream) {
 // same m as long as their maximum stays below m + kRaiseLog2 (log2 units), so
 // P = exp2(s - m) <= 2^kRaiseLog2 is exact in fp32 and in bf16 range and O, l
 // stay far from fp32 overflow.  A row whose scores jump higher (by more than
-// kRaiseLog2 * ln 2 within the row) marks its wave's 32 rows in raise_flags;
-// launch_fwd then reruns the 64-query tiles of those rows with the rescaling
-// kernel.
+// kRaiseLog2 * ln 2 within the row) marks its head in its wave's slot of
+// raise_flags; launch_fwd then reruns the 64-query tile of that head with the
+// rescaling kernel.
 //
 // SPLIT: few query rows over a long cached prefix (500 new tokens after 12000
 // are 128 workgroups; 16 are 4) do not fill the GPU.  Each tile's key tiles are
@@ -1488,11 +1589,21 @@ struct WideItem {
 };
 
 // Raise-flag slot of the 32-row wave whose first query is q (a multiple of
-// 32 / grp): the grp waves of a 32-query group take the group's head slots.
+// 32 / grp): the grp waves of a 32-query group take the slots of the group and
+// KV head, each with a bit per query head of its rows (raise_heads).
 __device__ __forceinline__ int64_t raise_slot(const g4_problem& p, int s, int q, int kvh,
                                               int grp) {
   const int nq32 = (p.seqlen_q + 31) / 32;
   return ((int64_t)s * nq32 + q / 32) * p.num_q_heads + kvh * grp + q % 32 * grp / 32;
+}
+
+// The query heads (bit = head of the group) with a marked row among a wave's 32:
+// row r, on lanes r and r + 32, is of head r % grp.
+__device__ __forceinline__ int raise_heads(bool marked, int grp) {
+  const unsigned long long m = __ballot(marked);
+  unsigned x = (unsigned)m | (unsigned)(m >> 32);
+  for (int o = 16; o >= grp; o >>= 1) x |= x >> o;
+  return (int)(x & ((1u << grp) - 1));
 }
 
 // Floats of a chunk's partial rows: 128 x D of O in register order (per wave,
@@ -1621,7 +1732,7 @@ __global__ void __launch_bounds__(256, 1) fwd_wide_kernel(FwdParams a) {
     s_cur = s_nxt;
   }
 
-  const bool raise_any = __ballot(ker.raise && q_valid) != 0;
+  const bool raise = ker.raise && q_valid;
   const float l_tot = ker.l_run + wave_xor32(ker.l_run);
   if constexpr (SPLIT) {
     float* part = a.part + ((int64_t)it.row_tile * a.kv_chunks + it.chunk) * kWidePartFloats<D>;
@@ -1634,18 +1745,19 @@ __global__ void __launch_bounds__(256, 1) fwd_wide_kernel(FwdParams a) {
         po[(b * 4 + r4) * 64] = f32x4{x[r4 * 4], x[r4 * 4 + 1], x[r4 * 4 + 2], x[r4 * 4 + 3]};
       }
     if (ker.h32 == 0) {
-      // (a sum of -1 marks the wave's rows for the rescaling pass)
+      // (a sum of -1 marks the row for the rescaling pass)
       float* ml = part + 128 * D + 2 * (ker.wave * 32 + l32);
       ml[0] = ker.m_run;
-      ml[1] = raise_any ? -1.f : l_tot;
+      ml[1] = raise ? -1.f : l_tot;
     }
     return;
   }
 
-  // Every wave reports whether its rows need the rescaling pass; the last
+  // Every wave reports the heads whose rows need the rescaling pass; the last
   // tile also clears the slots of its 32-query group past the tile.
+  const int heads = raise_heads(raise, grp);
   if (ker.lane == 0 && w_q / 32 * 32 < sq.lq)
-    a.raise_flags[raise_slot(p, s, w_q, kvh, grp)] = raise_any ? 1 : 0;
+    a.raise_flags[raise_slot(p, s, w_q, kvh, grp)] = heads;
   const int i1 = i0 + queries;
   if (i1 >= sq.lq && i1 % 32 != 0 && tid < grp && tid >= i1 % 32 * grp / 32)
     a.raise_flags[raise_slot(p, s, i1 / 32 * 32, kvh, grp) + tid] = 0;
@@ -1720,14 +1832,14 @@ __global__ void __launch_bounds__(256) merge_wide_kernel(FwdParams a) {
     raise |= l < 0.f;
     if (l > 0.f) mx = fmaxf(mx, m);
   }
-  const bool raise_any = __ballot(raise) != 0;
+  const int heads = raise_heads(raise && my_i < sq.lq, grp);
   if (quarter == 0 && tid == 0 && w_q / 32 * 32 < sq.lq)
-    a.raise_flags[raise_slot(p, it.s, w_q, it.kvh, grp)] = raise_any ? 1 : 0;
+    a.raise_flags[raise_slot(p, it.s, w_q, it.kvh, grp)] = heads;
   const int i1 = i0 + queries;
   if (quarter == 0 && w == 0 && i1 >= sq.lq && i1 % 32 != 0 && tid < grp &&
       tid >= i1 % 32 * grp / 32)
     a.raise_flags[raise_slot(p, it.s, i1 / 32 * 32, it.kvh, grp) + tid] = 0;
-  if (w_q >= sq.lq || raise_any) return;  // no such rows, or written by the rescaling pass
+  if (w_q >= sq.lq) return;  // (a marked head's rows are written again by the rescaling pass)
 
   // this workgroup's 32-column blocks of the wave's register-order partial
   constexpr int kB = D / 32 / 4;  // blocks
@@ -1867,12 +1979,13 @@ static hipError_t launch_fwd_cfg(const FwdParams& a, hipStream_t stream, bool fi
   if constexpr (D == 512)
     if (fixup) kern = fwd_kernel<D, BN, DSPLIT, NQG, VDOUBLE, 0, true, OCC>;
   const int variant = fixup ? 4 : meta;
+  const int lds = C::kLdsBytes + (fixup ? FixupScan::kLdsBytes : 0);
   static LdsAttr attr[5];
-  hipError_t e = attr[variant].ensure((const void*)kern, C::kLdsBytes);
+  hipError_t e = attr[variant].ensure((const void*)kern, lds);
   if (e != hipSuccess) return e;
   FwdParams b = a;
   b.doc_pass = doc_pass;
-  // (the fixup pass and the listed second document pass decode full-grid indices)
+  // (the rescaling pass and the listed second document pass decode full-grid indices)
   int64_t nblocks = fwd_grid(&b, C::kBM, !fixup && doc_pass != 2);
   if (nblocks <= 0) return hipSuccess;
   if (fixup) nblocks = std::min<int64_t>(nblocks, kFixupGrid);
@@ -1884,7 +1997,7 @@ static hipError_t launch_fwd_cfg(const FwdParams& a, hipStream_t stream, bool fi
     if (g <= 0) return hipErrorInvalidValue;
     nblocks = many ? g : nblocks;
   }
-  hipLaunchKernelGGL(kern, dim3((unsigned)nblocks), dim3(C::kNT), C::kLdsBytes, stream, b);
+  hipLaunchKernelGGL(kern, dim3((unsigned)nblocks), dim3(C::kNT), lds, stream, b);
   return hipGetLastError();
 }
 
@@ -1966,7 +2079,7 @@ hipError_t launch_fwd(const FwdParams& a, hipStream_t stream) {
   if (a.p.head_dim == 512) {
     if (meta_kind(a.p) != 0 || a.raise_flags == nullptr)
       return launch_fwd_cfg<512, 32, 2, 2, true>(a, stream);
-    // Fast pass, then the rescaling kernel on the 32-query groups it flagged.
+    // Fast pass, then the rescaling kernel on the 64-query tiles of the heads it flagged.
     hipError_t e = launch_fwd_wide<512>(a, stream);
     if (e != hipSuccess) return e;
     return launch_fwd_cfg<512, 32, 2, 2, true>(a, stream, /*fixup=*/true);

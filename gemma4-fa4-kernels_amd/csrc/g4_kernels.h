@@ -19,8 +19,8 @@ struct FwdParams {
   const int* span_hi;  // per K-stream token: last position of its vision span (or itself)
   int num_seqs;
   int ntq;             // query tiles per sequence (set by the launcher)
-  // Per (seq, 32-query group, head slot): row groups the fast pass cannot
-  // finish; the group's waves of the wide kernel take its KV head's slots.
+  // Per (seq, 32-query group, KV head, wave of the group's rows): the query
+  // heads, a bit each, with a row the fast pass cannot finish.
   int* raise_flags;
   // Split of a problem with document IDs over two launches (set by the
   // launcher): 0 every workgroup; 1 only workgroups whose queries and visited
