@@ -46,6 +46,9 @@ struct FwdParams {
   // Decode with equal parts (head dim 512): split_chunks parts, split_slots
   // slots of partial rows.  0: chunks of split_keys keys.
   int split_slots;
+  // Wide head-dim 512 forward: the sequences are of one length (set by the
+  // launcher).
+  int equal_order;
   // Wide head-dim 512 forward: key chunks per query tile (set by the launcher;
   // 1 unless `part` holds the chunks' partial rows).
   int kv_chunks;
