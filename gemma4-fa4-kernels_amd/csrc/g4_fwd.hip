@@ -1637,6 +1637,16 @@ __device__ __forceinline__ int raise_heads(bool marked, int grp) {
   return (int)(x & ((1u << grp) - 1));
 }
 
+// The MFMA fragments of a 32-row tile's rows.
+template <int CP, int NC, class RR>
+__device__ __forceinline__ void row_fragments(const RR& rrd, const char G4_LDS* t,
+                                              bf16x8 (&frag)[NC]) {
+  if constexpr (CP < NC) {
+    frag[CP] = rrd.template read<0, 0, CP>(t);
+    row_fragments<CP + 1>(rrd, t, frag);
+  }
+}
+
 // Floats of a chunk's partial rows: 128 x D of O in register order (per wave,
 // 1 KB per store), then the rows' maximum and sum.
 template <int D>
@@ -1706,14 +1716,25 @@ __global__ void __launch_bounds__(256, 1) fwd_wide_kernel(FwdParams a) {
   const bool q_valid = my_i < sq.lq;
   ker.lo_w = p.window > 0 ? my_a - p.window + 1 : -0x40000000;
   ker.hi_c = min(my_a, sq.lk - 1);
+  // Query fragments: each wave copies its rows whole into a quarter of the tile
+  // area and reads them as it reads K.  (Loaded from memory as fragments, every
+  // lane of an instruction is in another line, 64 cycles each: 9000 cycles, and
+  // as many for one query as for 16.)
+  const int nrows = max(min(32 >> gsh, sq.lq - w_q), 0) << gsh;  // the rows of this wave
   {
-    const __bf16* qrow = a.q + tok_off(sq, s, sq.qtok, min(my_i, sq.lq - 1), a.ql) +
-                         (int64_t)qh * a.ql.head_stride + ker.h32 * 8;
+    static_assert(C::kNW * 32 * D * 2 <= C::kLdsBytes && C::kCPR == 64, "staged rows");
+    char G4_LDS* stage = ker.smem + ker.wave * 32 * D * 2;
+    const __bf16* qbase = a.q + tok_off(sq, s, sq.qtok, w_q, a.ql) +
+                          (int64_t)(kvh * grp) * a.ql.head_stride;
+#pragma unroll 4
+    for (int r = 0; r < nrows; ++r)
+      b2l16(qbase + (r >> gsh) * a.ql.token_stride + (r & (grp - 1)) * a.ql.head_stride,
+            swz_slot(r, ker.lane) * 16u, stage + r * 1024);
+    vm_wait<0>();
+    row_fragments<0>(ker.krd, stage, ker.qf);
 #pragma unroll
-    for (int c = 0; c < K::kNC; ++c) {
-      bf16x8 x = ld_global16(qrow + c * 16);
-      ker.qf[c] = q_valid ? x : bf16x8{};
-    }
+    for (int c = 0; c < K::kNC; ++c) ker.qf[c] = q_valid ? ker.qf[c] : bf16x8{};
+    barrier_lds();  // every wave has read its rows
   }
   ker.m_run = kNegInf;
   ker.l_run = 0.f;
@@ -1802,7 +1823,6 @@ __global__ void __launch_bounds__(256, 1) fwd_wide_kernel(FwdParams a) {
   // area, 16-byte chunks swizzled by row.  (Stored as they lie, an item spent
   // 9-10 us after its loop; a 20-tile item's loop takes 40.)
   const float inv = l_tot > 0.f ? 1.f / l_tot : 0.f;
-  static_assert(C::kNW * 32 * D * 2 <= C::kLdsBytes, "staged rows");
   barrier_lds();  // every wave is done with the last tiles
   char G4_LDS* stage = ker.smem + ker.wave * 32 * D * 2;
 #pragma unroll
@@ -1817,15 +1837,23 @@ __global__ void __launch_bounds__(256, 1) fwd_wide_kernel(FwdParams a) {
   if (q_valid && ker.h32 == 0)
     a.lse[lse_off(p, sq, s, qh, my_i)] =
         l_tot > 0.f ? (ker.m_run + fast_log2(l_tot)) * kLn2 : kNegInf;
-#pragma unroll 8
-  for (int r = 0; r < 32; ++r) {
-    const int i = w_q + (r >> gsh);
-    if (i >= sq.lq) break;
-    __bf16* orow = a.o + tok_off(sq, s, sq.qtok, i, a.ol) +
-                   (int64_t)(kvh * grp + (r & (grp - 1))) * a.ol.head_stride;
-    static_assert(D * 2 == 64 * 16, "one 16-byte chunk per lane and row");
-    *(bf16x8*)(orow + ker.lane * 8) =
-        *(const bf16x8 G4_LDS*)(stage + r * D * 2 + (ker.lane ^ (r & 15)) * 16);
+  // Eight rows at a time, their LDS reads in flight together.
+  __bf16* const obase = a.o + tok_off(sq, s, sq.qtok, w_q, a.ol) +
+                        (int64_t)(kvh * grp) * a.ol.head_stride + ker.lane * 8;
+  static_assert(D * 2 == 64 * 16, "one 16-byte chunk per lane and row");
+  for (int r0 = 0; r0 < nrows; r0 += 8) {
+    bf16x8 v[8];
+#pragma unroll
+    for (int j = 0; j < 8; ++j)
+      v[j] = *(const bf16x8 G4_LDS*)(stage + (r0 + j) * D * 2 +
+                                     (ker.lane ^ ((r0 + j) & 15)) * 16);
+#pragma unroll
+    for (int j = 0; j < 8; ++j) {
+      const int r = r0 + j;
+      if (r < nrows)
+        *(bf16x8*)(obase + (r >> gsh) * a.ol.token_stride + (r & (grp - 1)) * a.ol.head_stride) =
+            v[j];
+    }
   }
 }
 
