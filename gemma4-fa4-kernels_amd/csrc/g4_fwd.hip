@@ -1958,14 +1958,19 @@ static int64_t wide_tiles(const g4_problem& p, int queries, int* compact) {
 
 // Key chunks per query tile of the wide forward: 1 (no split) or the count
 // whose rounds of workgroups over the 256 CUs are shortest, in key tiles of one
-// workgroup's walk: (chunk + kSetup) per round, plus the merge (its launch and
-// the partials written and read at about 4 TB/s, a key tile taking 1.2 us).
-// At least kMinTiles key tiles a chunk.
+// workgroup's walk (1.2 us): (chunk + kSetup) per round, plus the merge: its
+// launch, a chain of loads that grows with the chunks, and the partials written
+// and read, at about 10 TB/s as far as the caches hold them and 4 beyond.  At least
+// kMinTiles key tiles a chunk.  Measured, 32 heads of 4 KV heads, whole / split
+// us: 5 tokens over 200 keys 25.6 whole, 300 31 / 24, 512 42 / 27, 1000 65 / 30;
+// 48 over 450 41 / 30; 100 over 600 48 / 36; 300 over 1500 98 / 60; 500 over 2000
+// 129 / 91; 600 over 3000 186 whole.
 int wide_chunks(const g4_problem& p) {
   if (p.head_dim != 512 || (p.vision_ids != nullptr && p.bidirectional_vision) ||
       p.document_ids != nullptr)
     return 1;
-  constexpr int kSetup = 6, kMinTiles = 8, kCus = 256;
+  constexpr int kSetup = 6, kMinTiles = 2, kCus = 256;
+  constexpr double kTile = 1.2, kCached = 64e6;  // us; bytes of partials
   int compact;
   const int64_t items =
       wide_tiles(p, 128 / (p.num_q_heads / p.num_kv_heads), &compact) * p.num_kv_heads;
@@ -1974,10 +1979,14 @@ int wide_chunks(const g4_problem& p) {
                             : p.seqlen_k;
   const int64_t nt = (range + 31) / 32;
   int best = 1;
-  double best_cost = 0.9 * (double)((items + kCus - 1) / kCus) * (nt + kSetup);
+  double best_cost = (double)((items + kCus - 1) / kCus) * (nt + kSetup);
   for (int64_t n = 2; n <= 64 && n * kMinTiles <= nt && n * items <= 4 * kCus; ++n) {
-    const double cost = (double)((items * n + kCus - 1) / kCus) * ((nt + n - 1) / n + kSetup) + 5 +
-                        (double)(items * n) * kWidePartFloats<512> * 8 / 4e6 / 1.2;
+    const double bytes = (double)(items * n) * kWidePartFloats<512> * 4;
+    const double moved = 2 * (std::min(bytes, kCached) / 10e6 +
+                              std::max(bytes - kCached, 0.0) / 4e6);  // us
+    const double merge = 5 + 0.3 * n + moved / kTile;
+    const double cost =
+        (double)((items * n + kCus - 1) / kCus) * ((nt + n - 1) / n + kSetup) + merge;
     if (cost < best_cost) {
       best_cost = cost;
       best = (int)n;
