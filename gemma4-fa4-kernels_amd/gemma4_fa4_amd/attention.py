@@ -618,17 +618,19 @@ class _Plan:
         """The forward's workspace (None when it needs none) and its size.
 
         Phase 3 of g4_workspace_bytes, with room to split the keys over every
-        CU, where that is more than the forward needs; when that much (at most
-        256 MiB) cannot be had, what it needs.
+        CU, where that is more than the forward needs and the HBM is there
+        (``_room_for``), else what it needs.  The two routes sum over the keys in
+        different orders, so on a nearly full device the bits of O and LSE can
+        depend on how much HBM is free.
         """
         nbytes = self.workspace_bytes(0, prob)
         if self.head_dim == 512:
             split = self.workspace_bytes(3, prob)
-            if split > nbytes:
+            if split > nbytes and _room_for(split, device):
                 try:
                     return torch.empty(split, dtype=torch.uint8, device=device), split
                 except torch.OutOfMemoryError:
-                    pass
+                    _free_hbm(device)  # the reading was stale: later calls take this one
         # Most local forwards need no workspace (no vision IDs): the library
         # takes NULL for a zero-byte workspace, so none is allocated.
         return (torch.empty(nbytes, dtype=torch.uint8, device=device) if nbytes else None), nbytes
@@ -782,6 +784,21 @@ def _recent_free_hbm(device) -> int:
     if entry is not None and entry[2] is _free_hbm and time.monotonic() - entry[0] < _FREE_HBM_REUSE_S:
         return entry[1]
     return _free_hbm(device)
+
+
+def _room_for(nbytes: int, device) -> bool:
+    """Whether an optional workspace fits without the allocator giving up its cache.
+
+    An allocation that does not fit makes the caching allocator wait for the
+    device and release every block it holds before it raises, which costs far
+    more than the workspace would give.  So it is asked for only when it fits the
+    free HBM (one reading serves the calls of 20 ms, as in the checks above), or
+    the blocks that the allocator holds unused: a training process's allocator
+    usually holds nearly all of the HBM.
+    """
+    if nbytes <= _recent_free_hbm(device):
+        return True
+    return nbytes <= torch.cuda.memory_reserved(device) - torch.cuda.memory_allocated(device)
 
 
 def _preflight_metadata_workspace(plan: _Plan, device, free: int | None = None) -> int:
