@@ -548,9 +548,9 @@ class _Plan:
     # does not fit the guarded budget (GlobalBackwardBudgetExceeded).
     global_backward: bool = False
     # Additional bytes that fit at backward time beyond what the chosen route
-    # needs (0 with a pinned dS budget): the split dK/dV launch's partial tiles
-    # are taken from them (g4_workspace_bytes phase 2).
-    spare_bytes: int = 0
+    # needs (None with a pinned dS budget): the split dK/dV launch's partial
+    # tiles are taken from them (g4_workspace_bytes phase 2).
+    spare_bytes: int | None = None
     # Cumulative-array checks still to run before the first launch.
     pending: _CumulativeCheck | None = field(default=None, repr=False, compare=False)
     # Workspace sizes already asked of the library, by (phase, ds_budget): the
@@ -608,10 +608,14 @@ class _Plan:
 
     def _workspace(self, phase: int, device, prob: G4Problem | None = None) -> torch.Tensor:
         nbytes = max(self.workspace_bytes(phase, prob), 256)
-        if phase == 1 and self.spare_bytes > 0:
+        if phase == 1 and self.spare_bytes is not None:
             split = self.workspace_bytes(2, prob)
-            if split - nbytes <= self.spare_bytes:
-                nbytes = max(nbytes, split)
+            if split > nbytes and (split - nbytes <= self.spare_bytes
+                                   or _allocator_holds(split, device)):
+                try:
+                    return torch.empty(split, dtype=torch.uint8, device=device)
+                except torch.OutOfMemoryError:
+                    pass
         return torch.empty(nbytes, dtype=torch.uint8, device=device)
 
     def _forward_workspace(self, prob: G4Problem, device):
@@ -796,8 +800,10 @@ def _room_for(nbytes: int, device) -> bool:
     the blocks that the allocator holds unused: a training process's allocator
     usually holds nearly all of the HBM.
     """
-    if nbytes <= _recent_free_hbm(device):
-        return True
+    return nbytes <= _recent_free_hbm(device) or _allocator_holds(nbytes, device)
+
+
+def _allocator_holds(nbytes: int, device) -> bool:
     return nbytes <= torch.cuda.memory_reserved(device) - torch.cuda.memory_allocated(device)
 
 
@@ -877,12 +883,15 @@ def pin_backward_ds_budget(nbytes: int | None) -> int | None:
     ``None`` (the default) fits the budget to the free HBM at each forward and
     again at each backward: the dK/dV stage stores dS tiles while they fit, a
     single global sequence past that is striped, else the dQ stage recomputes S
-    and dP.  The recompute route sums dQ in another order, and the striped
-    route adds dK / dV over its stripes in fp32, so with the default the bits of
-    the gradients can depend on how much HBM is free.  A pinned budget fixes the
-    route: a negative value always recomputes, a positive one stores the tiles
-    (or stripes) that fit in that many bytes, 0 is the library's default cap
-    (16 GiB).  The global layers still raise
+    and dP; and a problem whose key tiles do not fill the GPU cuts its dK/dV work
+    over all CUs while 128 MiB more fit.  The recompute route sums dQ in another
+    order, and the striped and the cut routes add dK / dV in parts in fp32, so
+    with the default the bits of the gradients can depend on how much HBM is
+    free.  A pinned budget fixes the route: a negative value always recomputes, a
+    positive one stores the tiles (or stripes) that fit in that many bytes, 0 is
+    the library's default cap (16 GiB), and with any of them the dK/dV work is
+    not cut.  The pin does not reach the forward, whose key split at head dim 512
+    is taken while its workspace fits.  The global layers still raise
     ``GlobalBackwardBudgetExceeded`` when the pinned route does not fit the
     guarded budget.  A process-wide setting (not per thread).
     """
@@ -927,7 +936,7 @@ def _refit_backward(plan: _Plan, q, k, v) -> None:
     """
     free = _free_hbm(q.device)
     required = _fit_or_pin(plan, q, k, v, free)
-    plan.spare_bytes = 0 if _PINNED_DS_BUDGET is not None else \
+    plan.spare_bytes = None if _PINNED_DS_BUDGET is not None else \
         _global_backward_budget(free) - required
     if plan.global_backward:
         _check_global_backward_budget(required, free)

@@ -74,3 +74,68 @@ def test_forward_falls_back_and_reads_afresh_when_the_reading_was_stale(monkeypa
     hbm = _Hbm(monkeypatch, free=most, refuse_above=need)
     _, nbytes = plan._forward_workspace(plan.problem(), CPU)
     assert nbytes == need and hbm.asked[0] == most and hbm.readings == 2
+
+
+# ---- backward: the split dK/dV launch ----------------------------------------
+
+
+def _backward_plan():
+    q = torch.empty(1, 1000, 32, 512, dtype=torch.bfloat16)
+    k = torch.empty(1, 1000, 4, 512, dtype=torch.bfloat16)
+    plan = att._fixed_plan(q, k, g.GLOBAL_ATTENTION)
+    plan.global_backward = True
+    need, most = plan.workspace_bytes(1), plan.workspace_bytes(2)
+    assert most > need, "the problem is not split"
+    return plan, q, k, need, most
+
+
+def _free_for(budget):  # free bytes whose guarded budget is `budget`
+    return max(budget * 5 // 4 + 4, budget + 2 * 1024 ** 3)
+
+
+def _refit_and_ask(monkeypatch, beyond, **hbm_kw):
+    """Sizes asked for with ``beyond`` bytes free past what the backward needs."""
+    plan, q, k, need, most = _backward_plan()
+    free = _free_for(att._backward_additional_bytes(plan, q, k, k) + beyond)
+    hbm = _Hbm(monkeypatch, free=free, **hbm_kw)
+    att._refit_backward(plan, q, k, k)
+    plan._workspace(1, CPU)
+    return hbm.asked, need, most
+
+
+def test_backward_is_split_where_its_workspace_fits(monkeypatch):
+    _, _, _, need, most = _backward_plan()
+    asked, _, _ = _refit_and_ask(monkeypatch, most - need)
+    assert asked == [most]
+
+
+def test_backward_is_not_split_on_a_full_device(monkeypatch):
+    _, _, _, need, most = _backward_plan()
+    asked, _, _ = _refit_and_ask(monkeypatch, most - need - 1, reserved=most, allocated=1)
+    assert asked == [need]
+
+
+def test_backward_counts_the_blocks_that_the_allocator_holds(monkeypatch):
+    # A training process's allocator has taken nearly all of the HBM.
+    _, _, _, _, most = _backward_plan()
+    asked, _, _ = _refit_and_ask(monkeypatch, 0, reserved=most + 5, allocated=5)
+    assert asked == [most]
+
+
+def test_backward_falls_back_when_the_larger_workspace_is_refused(monkeypatch):
+    _, _, _, need, most = _backward_plan()
+    asked, _, _ = _refit_and_ask(monkeypatch, most, refuse_above=need)
+    assert asked == [most, need]
+
+
+@pytest.mark.parametrize("pin", [-1, 0, 1 << 34])
+def test_pinned_backward_is_never_split(monkeypatch, pin):
+    previous = g.pin_backward_ds_budget(pin)
+    try:
+        plan, q, k, _, most = _backward_plan()
+        hbm = _Hbm(monkeypatch, free=1 << 50, reserved=1 << 50)
+        att._refit_backward(plan, q, k, k)
+        plan._workspace(1, CPU)
+        assert hbm.asked == [plan.workspace_bytes(1)] and hbm.asked[0] < most
+    finally:
+        g.pin_backward_ds_budget(previous)
