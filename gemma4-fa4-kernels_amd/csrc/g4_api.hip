@@ -133,6 +133,21 @@ float* dkdv_split_ptr(const g4_problem& p, void* ws, size_t bytes) {
   const size_t own = bwd_ws_bytes(p), part = g4::dkdv_split_bytes(p);
   return part && bytes >= own + part ? (float*)((char*)ws + own) : nullptr;
 }
+// Workspace of a forward that splits its keys over every CU (phase 3).
+size_t fwd_split_ws_bytes(const g4_problem& p) {
+  if (!g4::split_bytes(p)) return fwd_ws_bytes(p) + g4::wide_split_bytes(p);
+  const size_t parts = g4::decode_bytes(p);
+  return fwd_ws_bytes(p) + (parts ? std::max(parts, g4::split_bytes(p)) - g4::split_bytes(p) : 0);
+}
+// Whether a forward's workspace holds the parts of that split.  A buffer of the
+// backward's size (phase 1 or 2) is taken as such: what it has beyond the
+// forward's needs is dS, whose size follows the dS budget, and the bits of O and
+// LSE must not.
+bool fwd_split_room(const g4_problem& p, size_t bytes) {
+  if (bytes < fwd_split_ws_bytes(p)) return false;
+  const size_t bwd = bwd_ws_bytes(p);
+  return bytes != bwd && (bytes != bwd + g4::kDkdvSplitBytes || g4::dkdv_split_bytes(p) == 0);
+}
 float* acc_ptr(const g4_problem& p, void* ws) {
   if (!g4::acc_bytes(p)) return nullptr;
   return (float*)((char*)sched_ptr(p, ws) + g4::kSchedBytes + g4::dq_list_bytes(p));
@@ -197,16 +212,16 @@ int fwd_impl(const g4_problem* p, const void* q, g4_layout ql, const void* k, g4
   g4::span_arrays(*p, ws, &a.span_lo, &a.span_hi);
   a.raise_flags = raise_flags_ptr(*p, ws);
   a.part = split_ptr(*p, ws);
+  const bool room = fwd_split_room(*p, ws_bytes);
   if (a.part != nullptr) {
     a.split_chunks = g4::split_chunks(*p, &a.split_keys);
     const int parts = g4::decode_parts(*p);
-    if (parts && ws_bytes >= fwd_ws_bytes(*p) - g4::split_bytes(*p) + g4::decode_bytes(*p)) {
+    if (parts && room) {
       a.split_chunks = parts;
       a.split_slots = parts + p->num_seqs * p->num_kv_heads;
     }
   }
-  if (const size_t wide = g4::wide_split_bytes(*p);
-      a.part == nullptr && wide && ws_bytes >= fwd_ws_bytes(*p) + wide)
+  if (a.part == nullptr && room && g4::wide_split_bytes(*p))
     a.part = (float*)((char*)ws + fwd_ws_bytes(*p));
   if (unsigned* dl = fwd_doc_list_ptr(*p, ws)) {
     a.doc_list_n = dl;
@@ -504,8 +519,7 @@ size_t dkdv_split_bytes(const g4_problem& p) {
   const double parts = std::min<double>(kSplitParts, std::max(1.0, total / kSplitMinPart));
   const double split = kSplitStep * total / parts + kSplitTileCost + kSplitSumSteps;
   if (whole <= 1.05 * split) return 0;
-  return 2 * (size_t)kSplitParts * kSplitSlotFloats * 4 +
-         align256((kSplitParts + 1) * sizeof(SplitCut));
+  return kDkdvSplitBytes;
 }
 size_t split_bytes(const g4_problem& p) {
   const int n = split_chunks(p, nullptr);
@@ -526,11 +540,7 @@ size_t g4_workspace_bytes(const g4_problem* p, int phase) {
   if (check_problem(p) != G4_OK) return 0;
   if (phase == 1) return bwd_ws_bytes(*p);
   if (phase == 2) return bwd_ws_bytes(*p) + g4::dkdv_split_bytes(*p);
-  if (phase == 3)
-    return fwd_ws_bytes(*p) +
-           (g4::split_bytes(*p) ? std::max(g4::decode_bytes(*p), g4::split_bytes(*p)) -
-                                      g4::split_bytes(*p)
-                                : g4::wide_split_bytes(*p));
+  if (phase == 3) return fwd_split_ws_bytes(*p);
   return fwd_ws_bytes(*p);
 }
 

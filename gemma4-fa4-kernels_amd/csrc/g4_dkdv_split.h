@@ -72,6 +72,11 @@ struct SplitCut {
   int kvh, s, kt, pad;
 };
 
+// Workspace: two slots of a partial tile per part, then the cuts.
+constexpr size_t kDkdvSplitBytes =
+    2 * (size_t)kSplitParts * kSplitSlotFloats * 4 +
+    ((kSplitParts + 1) * sizeof(SplitCut) + 255) / 256 * 256;
+
 // Most key tiles of a split problem: four items per CU, an item holding up to
 // two of them.
 constexpr int kSplitMaxTiles = 2 * 4 * kSplitParts;

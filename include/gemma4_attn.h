@@ -101,7 +101,9 @@ const char* g4_last_error(void);
  * Phase 3: phase 0 plus, for a forward whose query rows do not fill the GPU
  * over a long key range (a decode step; at head dim 512 a chunk of new tokens
  * after a cached prefix), room for more partial rows.  A forward given at least
- * that much splits its keys over all CUs and merges the parts. */
+ * that much splits its keys over all CUs and merges the parts.  A buffer of
+ * exactly the size of phase 1 or 2 is the backward's, and a forward in it does
+ * not split: the size follows ds_budget, and the bits of O and LSE do not. */
 size_t g4_workspace_bytes(const g4_problem* p, int phase);
 
 /*

@@ -73,3 +73,35 @@ def test_split_wide_forward_matches_the_oracle(hq, hkv, lq, lk, packed, window, 
                                          ck.tolist(), sliding_window=window,
                                          compute_dtype=torch.float64)
     check_forward(o, lse, o_ref.cpu(), l_ref.cpu(), local=False, label=label)
+
+
+@pytest.mark.parametrize("lq,lk,hq,hkv", [([2048], [2048], 8, 2), ([16], [4096], 32, 4),
+                                          ([1, 1], [3000, 900], 32, 4)])
+def test_forward_in_a_backward_workspace_is_not_split(lq, lk, hq, hkv):
+    """O and LSE of a forward given the backward's buffer do not follow its dS budget.
+
+    Such a buffer's room past the forward's needs is dS; with 16 GiB of budget, with
+    none and with the partial dK / dV tiles behind it, the forward is the one of the
+    smallest workspace to the bit, and phase 3 still splits.
+    """
+    from gemma4_fa4_amd import ops
+
+    print(f"forward in a backward workspace lq={lq} lk={lk} hq={hq}", flush=True)
+    q, k, v, _do, _dl = qkv(9990, sum(lq), sum(lk), hq, hkv, 512)
+    q, k, v = (t.to(DEV) for t in (q, k, v))
+    got = {}
+    for phase, budget in ((0, 0), (3, 0), (1, 0), (1, -1), (2, 0)):
+        plan = ops.make_plan(
+            num_seqs=len(lq), seqlen_q=max(lq), seqlen_k=max(lk), num_q_heads=hq,
+            num_kv_heads=hkv, head_dim=512, window=None, cu_q=cu(lq).to(DEV), cu_k=cu(lk).to(DEV),
+            total_q=sum(lq), total_k=sum(lk))
+        plan.ds_budget = budget
+        st = ops.Stages(plan, q, k, v, q, forward_only=True)
+        st.ws = torch.empty(plan.workspace_bytes(phase), dtype=torch.uint8, device=DEV).fill_(0xFF)
+        st.forward()
+        got[phase, budget] = st.o, st.lse
+    o, lse = got.pop((0, 0))
+    split = got.pop((3, 0))
+    assert not torch.equal(split[0], o)
+    for key, (o2, lse2) in got.items():
+        assert torch.equal(o2, o) and torch.equal(lse2, lse), key
