@@ -1024,24 +1024,40 @@ struct DecodeCfg {
   static constexpr int kLdsBytes = kLdsX + (kNW > 1 ? kNW * 4096 : 0);
 };
 
-// The key tiles of the segments, end to end: sequence-major, KV head, tile.
+// The key tiles of the segments, end to end: sequence-major, KV head, tile.  Of up
+// to 64 packed sequences lane s holds sequence s, so that the cumulative arrays
+// are read once and not again at each step from a position to its keys (about a
+// microsecond each time, with nothing else to do).
 struct DecodeMap {
   const g4_problem* p;
   int total;  // tiles of all segments
+  bool held;
+  int q0, k0, lq, lk, first, n, start;  // the lane's sequence
 
   struct Keys {
     int first, n;  // tiles a sequence's queries reach
   };
-  __device__ __forceinline__ Keys keys(int s) const {
-    int lq = p->seqlen_q, lk = p->seqlen_k;
-    if (p->cu_seqlens_q != nullptr) {
-      lq = p->cu_seqlens_q[s + 1] - p->cu_seqlens_q[s];
-      lk = p->cu_seqlens_k[s + 1] - p->cu_seqlens_k[s];
-    }
+  __device__ __forceinline__ Keys range(int lq, int lk) const {
     if (lq <= 0) return {0, 0};
     int lo, hi;
     query_tile_key_range(lk - lq, lk - 1, lk, p->window, -1, lo, hi);
     return {lo / 32, hi > lo ? (hi + 31) / 32 - lo / 32 : 0};
+  }
+  __device__ __forceinline__ Keys keys(int s) const {
+    if (held) return {__builtin_amdgcn_readlane(first, s), __builtin_amdgcn_readlane(n, s)};
+    if (p->cu_seqlens_q == nullptr) return range(p->seqlen_q, p->seqlen_k);
+    return range(p->cu_seqlens_q[s + 1] - p->cu_seqlens_q[s],
+                 p->cu_seqlens_k[s + 1] - p->cu_seqlens_k[s]);
+  }
+  __device__ __forceinline__ Seq seq(int s) const {
+    if (!held) return resolve_seq(*p, s);
+    Seq r;
+    r.packed = true;
+    r.lq = __builtin_amdgcn_readlane(lq, s);
+    r.lk = __builtin_amdgcn_readlane(lk, s);
+    r.qtok = __builtin_amdgcn_readlane(q0, s);
+    r.ktok = __builtin_amdgcn_readlane(k0, s);
+    return r;
   }
   __device__ __forceinline__ static int scan(int x) {
     const int lane = __lane_id();
@@ -1054,8 +1070,23 @@ struct DecodeMap {
   }
   __device__ __forceinline__ void init(const g4_problem& prob) {
     p = &prob;
+    held = p->cu_seqlens_q != nullptr && p->num_seqs <= 64;
     if (p->cu_seqlens_q == nullptr) {
       total = keys(0).n * p->num_seqs * p->num_kv_heads;
+      return;
+    }
+    if (held) {
+      const int s = min((int)__lane_id(), p->num_seqs - 1);
+      q0 = p->cu_seqlens_q[s];
+      k0 = p->cu_seqlens_k[s];
+      lq = p->cu_seqlens_q[s + 1] - q0;
+      lk = p->cu_seqlens_k[s + 1] - k0;
+      const Keys r = range(lq, lk);
+      first = r.first;
+      n = (int)__lane_id() < p->num_seqs ? r.n : 0;
+      const int end = scan(n);
+      start = (end - n) * p->num_kv_heads;
+      total = __builtin_amdgcn_readlane(end, 63) * p->num_kv_heads;
       return;
     }
     int sum = 0;
@@ -1063,32 +1094,38 @@ struct DecodeMap {
     total = __builtin_amdgcn_readlane(scan(sum), 63) * p->num_kv_heads;
   }
   // Sequence s that holds position pos < total, and its first position.
-  __device__ __forceinline__ void find(int pos, int& s, int& start) const {
+  __device__ __forceinline__ void find(int pos, int& s, int& first_pos) const {
     const int hkv = p->num_kv_heads;
     if (p->cu_seqlens_q == nullptr) {
       const int per = keys(0).n * hkv;
       s = pos / per;
-      start = s * per;
+      first_pos = s * per;
       return;
     }
-    start = 0;
+    if (held) {
+      s = __builtin_amdgcn_readfirstlane(__popcll(__ballot(start + n * hkv <= pos)));
+      first_pos = __builtin_amdgcn_readlane(start, s);
+      return;
+    }
+    first_pos = 0;
     for (int base = 0; base < p->num_seqs; base += 64) {
       const int mine = base + (int)__lane_id();
       const int cnt = mine < p->num_seqs ? keys(mine).n * hkv : 0;
-      const int incl = scan(cnt) + start;
+      const int incl = scan(cnt) + first_pos;
       const int end = __builtin_amdgcn_readlane(incl, 63);
       if (pos < end) {
         const int at = __builtin_amdgcn_readfirstlane(__popcll(__ballot(incl <= pos)));
         s = base + at;
-        start = __builtin_amdgcn_readlane(incl - cnt, at);
+        first_pos = __builtin_amdgcn_readlane(incl - cnt, at);
         return;
       }
-      start = end;
+      first_pos = end;
     }
     s = p->num_seqs;  // (pos >= total)
   }
   // First position of sequence s.
   __device__ __forceinline__ int start_of(int s) const {
+    if (held) return __builtin_amdgcn_readlane(start, s);
     if (p->cu_seqlens_q == nullptr) return s * keys(0).n * p->num_kv_heads;
     int sum = 0;
     for (int t = __lane_id(); t < s; t += 64) sum += keys(t).n;
@@ -1253,7 +1290,7 @@ __global__ void __launch_bounds__(D / 4) fwd_decode_kernel(FwdParams a) {
     const int kvh = (pos - start) / keys.n;
     const int t_lo = (pos - start) - kvh * keys.n;
     const int t_hi = min(keys.n, t_lo + end - pos);
-    ker.sq = resolve_seq(p, s);
+    ker.sq = map.seq(s);
     const Seq& sq = ker.sq;
     ker.lq = sq.lq;
     ker.off = sq.lk - sq.lq;
@@ -1328,12 +1365,12 @@ __global__ void __launch_bounds__(256) merge_decode_kernel(FwdParams a) {
   const int quarter = blockIdx.x % Q;
   const int seg = blockIdx.x / Q / rows, r = blockIdx.x / Q % rows;
   const int s = seg / p.num_kv_heads, kvh = seg % p.num_kv_heads;
-  const Seq sq = resolve_seq(p, s);
+  DecodeMap map;
+  map.init(p);
+  const Seq sq = map.seq(s);
   if (r >= grp * sq.lq) return;
   const int qh = kvh * grp + r / sq.lq, qi = r % sq.lq;
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  DecodeMap map;
-  map.init(p);
   const int tiles = map.keys(s).n;
   int g0 = 0, n = 0;
   if (tiles > 0) {
