@@ -46,7 +46,12 @@ __device__ __forceinline__ float wave_sum(float x) {
 // with strides below 2^32 elements the row index is split with multipliers from
 // the host and an offset is three 32 x 32 + 64 bit multiply-adds (NARROW);
 // anything larger keeps the 64-bit form, and so does the backward, where it
-// made no difference (32.3 us for 32768 rows of 512 either way).
+// made no difference (32.3 us for 32768 rows of 512 either way).  So do
+// kWideRows rows or more with K in fp32: they no longer fit the caches and are
+// bound by HBM (4 TB/s), which the faster issue disturbs (rows of 512, 64-bit /
+// NARROW us: 65536 71.9 / 71.8, 131072 135.6 / 137.5, 262144 264 / 267, 524288
+// 543 / 564; K in bf16 262144 203 / 201).
+constexpr int64_t kWideRows = int64_t(1) << 17;
 struct RowMap {
   uint32_t heads_mul, seq_mul;
   int heads_shift, seq_shift;
@@ -70,7 +75,7 @@ template <class... L>
 RowMap row_map(const g4_kv_prep& p, const L&... layouts) {
   RowMap m{};
   const int64_t rows = (int64_t)p.num_batches * p.seqlen * p.num_heads;
-  m.narrow = rows < (int64_t(1) << 31) && (p.cs_batch_stride >> 32) == 0 &&
+  m.narrow = rows < (p.k_fp32 ? kWideRows : int64_t(1) << 31) && (p.cs_batch_stride >> 32) == 0 &&
              (narrow_layout(layouts) && ...);
   if (m.narrow) {
     division((uint32_t)p.num_heads, m.heads_mul, m.heads_shift);

@@ -1,5 +1,8 @@
 """Row preparation at the edges of its row split and of its two address forms.
 
+K in fp32 takes the 64-bit address form from 2^17 rows on; halves of such a call
+take the other one and must give the same bits.
+
 Head dim 256 takes two rows per wave, so odd row counts end in half a wave; row
 indexes are split with multipliers, so head counts and lengths that are and are
 not powers of two are covered; a batch stride of 2^32 elements (one batch, so
@@ -67,3 +70,22 @@ def test_row_preparation_edges(d, b, h, s, rotary):
         prepare_rows_into(_wide(zd), weight=w.to(DEV), rotary_dim=rotary, eps=EPS, k=_wide(k2),
                           v=_wide(v2), **tables)
         assert torch.equal(k, k2) and torch.equal(v, v2)
+
+
+@pytest.mark.parametrize("heads,s", [(4, 32768), (4, 32767), (3, 43691)])
+def test_large_fp32_preparation_matches_its_halves(heads, s):
+    import gemma4_fa4_amd as g4
+
+    g = torch.Generator(device=DEV).manual_seed(s)
+    z = torch.randn(1, heads, s, 512, generator=g, device=DEV).to(torch.bfloat16)
+    w = torch.rand(512, generator=g, device=DEV) + 0.5
+    ang = torch.rand(s, 128, generator=g, device=DEV) * 6
+    cos, sin = torch.cos(ang), torch.sin(ang)
+    with torch.no_grad():
+        whole = g4.prepare_global_kv_from_projection_source(z, k_norm_weight=w, cos=cos, sin=sin)
+        at = s // 2
+        for part in (slice(0, at), slice(at, s)):
+            got = g4.prepare_global_kv_from_projection_source(
+                z[:, :, part], k_norm_weight=w, cos=cos[part], sin=sin[part])
+            for x, y in zip(whole, got):
+                assert torch.equal(x[:, :, part], y)
