@@ -1,4 +1,7 @@
-"""Vision spans of up to 4096 K tokens: one workgroup instead of the six passes.
+"""Vision spans of few K tokens: one workgroup instead of the six passes.
+
+One sequence takes it up to 4096 tokens, several up to 3584 in the backward's
+form (the key tiles' ranges too, as here) and 1792 in the forward's.
 
 The same sequences are scheduled alone (one workgroup, table in LDS) and with a
 text sequence appended that takes the batch past the limit (the passes over the
@@ -35,6 +38,8 @@ def _ranges(lq, lk, vis, docs):
     (2, [4096], [4096], True),
     (3, [1, 1300], [1, 2500], False),
     (4, [9] * 256, [16] * 256, True),
+    (6, [9] * 256, [14] * 256, True),
+    (7, [500, 700], [1000, 2584], True), (8, [500, 700], [1000, 2585], True),
     (5, [5] * 300, [5] * 300, False),  # too many sequences: the passes either way
 ])
 def test_small_spans_match_the_passes(seed, lq, lk, with_docs):
