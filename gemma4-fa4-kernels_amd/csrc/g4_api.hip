@@ -130,8 +130,9 @@ size_t bwd_ws_bytes(const g4_problem& p) {
 // The split dK/dV launch's partial tiles, when the caller's workspace holds
 // them beyond the backward's own needs (g4_workspace_bytes phase 2).
 float* dkdv_split_ptr(const g4_problem& p, void* ws, size_t bytes) {
-  const size_t own = bwd_ws_bytes(p), part = g4::dkdv_split_bytes(p);
-  return part && bytes >= own + part ? (float*)((char*)ws + own) : nullptr;
+  const size_t own = bwd_ws_bytes(p);
+  const bool split = bytes >= own + g4::kDkdvSplitBytes && g4::dkdv_split_bytes(p) > 0;
+  return split ? (float*)((char*)ws + own) : nullptr;
 }
 // Workspace of a forward that splits its keys over every CU (phase 3).
 size_t fwd_split_ws_bytes(const g4_problem& p) {
@@ -450,13 +451,13 @@ size_t decode_bytes(const g4_problem& p) {
                   (p.head_dim + 2) * 4);
 }
 // Split dK/dV launch (g4_dkdv_split.h) against the launch by whole key tiles
-// (head dim 512: pairs of tiles) on the 256 CUs, in steps of the longest chain
-// of one CU (about 2.2 us at head dim 512, 1.9 us at 256).
+// (head dim 512: pairs of tiles) on the 256 CUs.  Head dim 256, several
+// sequences: SplitTiles256.  Else in steps of the longest chain of one CU (about
+// 2.2 us at head dim 512, 1.9 us at 256):
 //  - Whole tiles of equal sequences: full rounds of the costliest item.  Of
 //    unequal packed sequences: the costliest item while every item has a CU,
 //    else the average plus part of the costliest item (measured: head dim 512,
-//    16 x 1000 tokens 1.26 x the average, [6000, 6000] 1.5 x; head dim 256,
-//    16 x 500 tokens 1.65 x).
+//    16 x 1000 tokens 1.26 x the average, [6000, 6000] 1.5 x).
 //  - Split: the average, each step 1.3 x as long (the parts walk different query
 //    rows at a time, so Q and dO come from beyond the L2: 2.7-2.9 us against
 //    2.2-2.4 at 4096-8192 tokens), plus set-up and the sum.
@@ -483,6 +484,20 @@ size_t dkdv_split_bytes(const g4_problem& p) {
   const int64_t items = (int64_t)p.num_seqs * per_seq * p.num_kv_heads;
   if (items > 4 * kSplitParts) return 0;
   const int grp = p.num_q_heads / p.num_kv_heads;
+  const int64_t rest_k = p.total_k - p.seqlen_k;  // packed: keys of the other sequences
+  const int64_t rest_q = std::max<int64_t>(p.total_q - p.seqlen_q, 0);
+  if (p.head_dim == 256 && p.num_seqs > 1) {
+    const int64_t n = p.num_seqs - 1;
+    const int lk = packed ? (int)std::clamp<int64_t>(rest_k / n, 0, p.seqlen_k) : p.seqlen_k;
+    const int lq = packed ? (int)std::min<int64_t>(rest_q / n, lk) : p.seqlen_q;
+    const bool images = p.vision_ids != nullptr && p.bidirectional_vision;
+    SplitTiles256 tiles;
+    tiles.nseq = p.num_seqs;
+    tiles.hkv = p.num_kv_heads;
+    tiles.fill(0, p.seqlen_q, p.seqlen_k, p.window, grp, images);
+    tiles.fill(1, lq, lk, p.window, grp, images);
+    return tiles.whole() > 1.05 * tiles.split() ? kDkdvSplitBytes : 0;
+  }
   SplitSeq q;  // a sequence of the largest lengths
   q.init(p.seqlen_q, p.seqlen_k, bn, p.window, grp);
   double longest = 0;  // item
@@ -493,12 +508,10 @@ size_t dkdv_split_bytes(const g4_problem& p) {
     longest = std::max(longest, c);
   }
   double total, whole;
-  const int64_t rest_k = p.total_k - p.seqlen_k;  // packed: keys of the other sequences
   if (packed && p.num_seqs > 1 && rest_k < (int64_t)(p.num_seqs - 1) * p.seqlen_k) {
     // the others' lengths are on the device: between as many as fit of the
     // largest length and all equal
     const double most = (double)p.total_k / p.seqlen_k * q.before((int)nt);
-    const int64_t rest_q = std::max<int64_t>(p.total_q - p.seqlen_q, 0);
     SplitSeq o;
     o.init((int)std::min(rest_q / (p.num_seqs - 1), rest_k / (p.num_seqs - 1)),
            (int)(rest_k / (p.num_seqs - 1)), bn, p.window, grp);
@@ -508,11 +521,9 @@ size_t dkdv_split_bytes(const g4_problem& p) {
     total = (double)p.num_seqs * p.num_kv_heads * q.before((int)nt);
   }
   if (packed && p.num_seqs > 1) {
-    // items that exist: a pair of 64-key tiles or one 128-key tile
+    // items that exist: pairs of 64-key tiles
     const double real = (double)p.total_k / 128 * p.num_kv_heads;
-    whole = real <= kSplitParts
-                ? longest
-                : (p.head_dim == 512 ? 1.0 : 1.4) * total / kSplitParts + 0.6 * longest;
+    whole = real <= kSplitParts ? longest : total / kSplitParts + 0.6 * longest;
   } else {
     whole = (double)((items + kSplitParts - 1) / kSplitParts) * longest;
   }

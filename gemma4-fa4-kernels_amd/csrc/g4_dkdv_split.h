@@ -15,6 +15,8 @@
 // alone, so results repeat bitwise.
 #pragma once
 
+#include <algorithm>
+
 #include "g4_kernels.h"
 
 namespace g4 {
@@ -61,6 +63,100 @@ struct SplitSeq {
     int rows = windowed ? split_ramp(kt, m, h0) - split_ramp(kt, m, h0 - nrows) : kt * nrows;
     rows -= split_ramp(kt, m, -e);
     return rows * grp + kt * kSplitTileCost;
+  }
+};
+
+// Head dim 256: the two launches' times from their schedules.  An average over
+// the CUs does not tell them apart (packed sequences of one length, split /
+// whole: 8 x 300 tokens 0.78, 12 x 300 1.21, 16 x 300 0.93): which items share a
+// CU, and how many tiles a part touches, follow from the counts, so both
+// schedules are walked.  The sequences are the longest first, then the others at
+// their mean length (their own are on the device); with vision IDs every
+// sequence is taken to hold one image of at most 700 tokens per 4000, which
+// lengthens the tiles it lies in.  Both against 138 measured problems of 2 to 64
+// sequences: 5% and 6%.
+struct SplitTiles256 {
+  static constexpr int kMax = 4 * kSplitParts;  // items of a problem that may split
+  int steps[2][kMax];  // of a key tile of the longest sequence, of another one
+  int nt[2];           // their key tiles
+  int nseq, hkv;
+
+  void fill(int which, int lq, int lk, int window, int grp, bool images) {
+    const int off = lk - lq, nrows = lq > 0 ? (lq + 31) / 32 : 0;
+    nt[which] = std::min((lk + 127) / 128, kMax);
+    for (int t = 0; t < nt[which]; ++t) {
+      int lo = std::max(128 * t - off, 0) >> 5;
+      const int last = std::min(128 * t + 127, lk - 1);  // key
+      const int hi = window > 0 ? std::min(nrows, ((last + window - 1 - off) >> 5) + 1) : nrows;
+      if (images) {
+        const int size = std::min(lk / 2, 700);
+        for (int at = lk / 4; at + lk / 2 <= lk && at <= last; at += 4000)
+          if (at + size > 128 * t) lo = std::min(lo, std::max(at - off, 0) >> 5);
+      }
+      steps[which][t] = std::max(hi - lo, 0) * grp;
+    }
+  }
+  int tile_steps(int s, int t) const { return steps[s > 0][t]; }
+
+  // Whole tiles, one workgroup each.  An XCD takes a run of the items and the
+  // hardware deals it to four shader engines of eight CUs in turn, in order: an
+  // item waits for a CU of its engine, and the later ones for it.
+  double whole() const {
+    const int per_kvh = nseq * nt[0], items = per_kvh * hkv;
+    double worst = 0;
+    for (int x = 0; x < (hkv % 8 == 0 ? 1 : 8); ++x) {
+      const int lo = x * (items / 8) + std::min(x, items % 8);
+      const int hi = lo + items / 8 + (x < items % 8 ? 1 : 0);
+      double busy[4][8] = {}, now = 0;
+      for (int i = lo; i < hi; ++i) {
+        const int rank = i % per_kvh, s = rank / nt[0], r = rank % nt[0];
+        const int t = r & 1 ? r >> 1 : nt[0] - 1 - (r >> 1);  // zigzag
+        double* cu = std::min_element(busy[(i - lo) & 3], busy[(i - lo) & 3] + 8);
+        now = std::max(now, *cu);
+        *cu = now + (t < nt[s > 0] ? tile_steps(s, t) + 7 : 0.3);
+        worst = std::max(worst, *cu);
+      }
+    }
+    return 1.88 * worst - 5;  // us
+  }
+  // Equal parts: a tile that a part touches costs it five steps, whether it runs
+  // all of it or not.
+  double split() const {
+    int cost = 0;
+    for (int s = 0; s < nseq; ++s)
+      for (int t = 0; t < nt[s > 0]; ++t) cost += tile_steps(s, t) + kSplitTileCost;
+    if (cost == 0) return 0;
+    const int64_t total = (int64_t)cost * hkv;
+    const int n = (int)std::min<int64_t>(kSplitParts, std::max<int64_t>(total / kSplitMinPart, 1));
+    const int walk = n % hkv == 0 ? n / hkv : n;  // (then the KV heads' parts are alike)
+    int s = 0, t = 0, worst = 0;
+    int64_t at = 0;  // where tile (s, t) begins
+    while (nt[s > 0] == 0) ++s;
+    for (int g = 0; g < walk; ++g) {
+      const int64_t from = total * g / n, to = total * (g + 1) / n;
+      int sum = 0;
+      for (;;) {
+        const int c = tile_steps(s, t);
+        const int64_t end = at + c + kSplitTileCost;
+        int lo = (int)std::max<int64_t>(from - at - kSplitTileCost, 0);
+        int hi = (int)std::min<int64_t>(std::max<int64_t>(to - at - kSplitTileCost, 0), c);
+        if (lo < kSplitMinSteps) lo = 0;
+        if (hi < kSplitMinSteps && to < end) hi = 0;
+        if (lo > 0 && c - lo < kSplitMinSteps) lo = c;
+        if (c - hi < kSplitMinSteps) hi = c;
+        if (hi > lo || (lo == 0 && hi == c)) sum += hi - lo + kSplitTileCost;
+        if (to < end) break;
+        at = end;
+        ++t;
+        while (t >= nt[s > 0]) {
+          t = 0;
+          if (++s == nseq) s = 0;  // the next KV head
+        }
+        if (at >= to) break;
+      }
+      worst = std::max(worst, sum);
+    }
+    return 2.48 * worst + 10;  // us
   }
 };
 
