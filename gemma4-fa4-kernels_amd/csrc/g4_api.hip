@@ -145,7 +145,7 @@ size_t fwd_split_ws_bytes(const g4_problem& p) {
 // forward's needs is dS, whose size follows the dS budget, and the bits of O and
 // LSE must not.
 bool fwd_split_room(const g4_problem& p, size_t bytes) {
-  if (bytes < fwd_split_ws_bytes(p)) return false;
+  if (p.head_dim != 512 || bytes < fwd_split_ws_bytes(p)) return false;
   const size_t bwd = bwd_ws_bytes(p);
   return bytes != bwd && (bytes != bwd + g4::kDkdvSplitBytes || g4::dkdv_split_bytes(p) == 0);
 }

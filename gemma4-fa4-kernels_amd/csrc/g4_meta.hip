@@ -285,13 +285,14 @@ static_assert(kSmallLds <= 160 * 1024, "LDS budget");
 // K tokens up to which the one workgroup pays.  With several sequences every token
 // is searched for its own, six steps for 64 of them, and the passes do that on
 // many CUs: the whole forward, passes / one workgroup us, 8 sequences of 192
-// tokens 35.9 / 34.9, of 256 48.5 / 48.9, of 512 91.8 / 95.2; 64 of 24 41.3 / 40.3,
-// of 32 43.6 / 44.4, of 64 65.2 / 72.6; one sequence of 4096 197.0 / 196.8.  The
-// backward's passes are six: forward and backward of 64 x 48 229 / 210, 64 x 56
-// 240 / 240, 64 x 64 250 / 256, 8 x 512 474 / 478.
+// tokens 35.9 / 34.9, of 256 48.5 / 48.9, of 320 64.1 / 64.0, of 512 91.8 / 95.2; 64 of 24 41.3 /
+// 40.3, of 40 55.8 / 56.4, of 64 65.2 / 72.6; one sequence of 4096 197.0 / 196.8.
+// A short training call waits for its launches: forward and backward of 4 x 500
+// 214 / 202.  The backward's passes are six: forward and backward of 64 x 48 229 /
+// 210, 64 x 56 240 / 240, 64 x 64 250 / 256, 8 x 512 474 / 478.
 int small_span_tokens(const g4_problem& p, bool query_reach) {
   if (p.num_seqs == 1) return kSmallTokens;
-  return p.num_seqs > kSmallSeqs ? 0 : query_reach ? 3584 : 1792;
+  return p.num_seqs > kSmallSeqs ? 0 : query_reach ? 3584 : 2560;
 }
 
 __global__ void __launch_bounds__(kReachChunk) span_small_kernel(g4_problem p, SpanWs out, int tk,

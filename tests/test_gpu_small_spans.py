@@ -1,7 +1,7 @@
 """Vision spans of few K tokens: one workgroup instead of the six passes.
 
 One sequence takes it up to 4096 tokens, several up to 3584 in the backward's
-form (the key tiles' ranges too, as here) and 1792 in the forward's.
+form (the key tiles' ranges too, as here) and 2560 in the forward's.
 
 The same sequences are scheduled alone (one workgroup, table in LDS) and with a
 text sequence appended that takes the batch past the limit (the passes over the
