@@ -551,6 +551,8 @@ class _Plan:
     # needs (None with a pinned dS budget): the split dK/dV launch's partial
     # tiles are taken from them (g4_workspace_bytes phase 2).
     spare_bytes: int | None = None
+    # The free-HBM reading of the forward's checks, if they took one.
+    free_bytes: int | None = None
     # Cumulative-array checks still to run before the first launch.
     pending: _CumulativeCheck | None = field(default=None, repr=False, compare=False)
     # Workspace sizes already asked of the library, by (phase, ds_budget): the
@@ -630,7 +632,7 @@ class _Plan:
         nbytes = self.workspace_bytes(0, prob)
         if self.head_dim == 512:
             split = self.workspace_bytes(3, prob)
-            if split > nbytes and _room_for(split, device):
+            if split > nbytes and _room_for(split, device, self.free_bytes):
                 try:
                     return torch.empty(split, dtype=torch.uint8, device=device), split
                 except torch.OutOfMemoryError:
@@ -790,17 +792,19 @@ def _recent_free_hbm(device) -> int:
     return _free_hbm(device)
 
 
-def _room_for(nbytes: int, device) -> bool:
+def _room_for(nbytes: int, device, free: int | None = None) -> bool:
     """Whether an optional workspace fits without the allocator giving up its cache.
 
     An allocation that does not fit makes the caching allocator wait for the
     device and release every block it holds before it raises, which costs far
     more than the workspace would give.  So it is asked for only when it fits the
-    free HBM (one reading serves the calls of 20 ms, as in the checks above), or
-    the blocks that the allocator holds unused: a training process's allocator
-    usually holds nearly all of the HBM.
+    free HBM (``free``, this call's reading, else one of the last 20 ms), or the
+    blocks that the allocator holds unused: a training process's allocator usually
+    holds nearly all of the HBM.
     """
-    return nbytes <= _recent_free_hbm(device) or _allocator_holds(nbytes, device)
+    if free is None:
+        free = _recent_free_hbm(device)
+    return nbytes <= free or _allocator_holds(nbytes, device)
 
 
 def _allocator_holds(nbytes: int, device) -> bool:
@@ -911,7 +915,7 @@ def _fit_or_pin(plan: _Plan, q, k, v, free: int) -> int:
 
 def _preflight_backward(plan: _Plan, q, k, v) -> None:
     plan.global_backward = True
-    free = _recent_free_hbm(q.device)
+    plan.free_bytes = free = _recent_free_hbm(q.device)
     required = _fit_or_pin(plan, q, k, v, free)
     _check_global_backward_budget(required, free)
 
@@ -942,7 +946,8 @@ def _refit_backward(plan: _Plan, q, k, v) -> None:
         _check_global_backward_budget(required, free)
 
 
-def _preflight_forward_outputs(q: torch.Tensor) -> None:
+def _preflight_forward_outputs(q: torch.Tensor) -> int:
+    """The forward's outputs against free HBM; returns the reading."""
     out_bytes = q.numel() * q.element_size()
     lse_bytes = q.numel() // q.shape[-1] * 4
     required = 2 * (out_bytes + lse_bytes)
@@ -952,6 +957,7 @@ def _preflight_forward_outputs(q: torch.Tensor) -> None:
             f"forward outputs require about {required} bytes, above 80% of the {free} "
             "currently free HBM bytes"
         )
+    return free
 
 
 def _requires_backward(*tensors) -> bool:
@@ -1049,8 +1055,10 @@ def fa4_local_varlen_forward(
 def fa4_global_forward_only(q, k, v, *, spec: AttentionLayerSpec = GLOBAL_ATTENTION):
     """Fixed/rectangular global d512 forward without autograd (lower-right causal)."""
     _validate_global_forward_only_bshd(q, k, v, spec)
-    _preflight_forward_outputs(q)
-    return _fixed_plan(q, k, spec).forward(q, k, v)
+    free = _preflight_forward_outputs(q)
+    plan = _fixed_plan(q, k, spec)
+    plan.free_bytes = free
+    return plan.forward(q, k, v)
 
 
 def fa4_global_varlen_forward_only(
@@ -1070,8 +1078,10 @@ def fa4_global_varlen_forward_only(
     )
 
     def prepare():
-        _preflight_forward_outputs(q)
-        return _packed_plan(q, k, cu_seqlens_q, cu_seqlens_k, max_seqlen_q, max_seqlen_k, spec)
+        free = _preflight_forward_outputs(q)
+        plan = _packed_plan(q, k, cu_seqlens_q, cu_seqlens_k, max_seqlen_q, max_seqlen_k, spec)
+        plan.free_bytes = free
+        return plan
 
     return _run_checked(q, k, v, check, prepare, autograd=False)
 
@@ -1098,7 +1108,7 @@ def fa4_global_varlen_forward(
         if _requires_backward(q, k, v):
             _preflight_backward(plan, q, k, v)
         else:
-            _preflight_forward_outputs(q)
+            plan.free_bytes = _preflight_forward_outputs(q)
         return plan
 
     return _run_checked(q, k, v, check, prepare)
@@ -1111,5 +1121,5 @@ def fa4_global_text_forward(q, k, v, *, spec: AttentionLayerSpec = GLOBAL_ATTENT
     if _requires_backward(q, k, v):
         _preflight_backward(plan, q, k, v)
     else:
-        _preflight_forward_outputs(q)
+        plan.free_bytes = _preflight_forward_outputs(q)
     return _run(q, k, v, plan)
