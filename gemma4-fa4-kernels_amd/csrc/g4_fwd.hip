@@ -1021,17 +1021,19 @@ struct DecodeCfg {
   static constexpr int kLdsK = 0;
   static constexpr int kLdsV = kTile;
   static constexpr int kLdsX = 2 * kTile;  // partial S of each wave
-  static constexpr int kLdsBytes = kLdsX + (kNW > 1 ? kNW * 4096 : 0);
+  static constexpr int kLdsBytes = kLdsX + kNW * 4096;
+  static_assert(kNW == 2, "each wave adds the one other slice's partial S");
 };
 
 // The key tiles of the segments, end to end: sequence-major, KV head, tile.  Of up
 // to 64 packed sequences lane s holds sequence s, so that the cumulative arrays
 // are read once and not again at each step from a position to its keys (about a
-// microsecond each time, with nothing else to do).
+// microsecond each time, with nothing else to do).  (HELD at compile time: tested
+// in the kernel it cost one unpacked 8000-token cache 0.5 us of 26.8.)
+template <bool HELD>
 struct DecodeMap {
   const g4_problem* p;
   int total;  // tiles of all segments
-  bool held;
   int q0, k0, lq, lk, first, n, start;  // the lane's sequence
 
   struct Keys {
@@ -1044,13 +1046,14 @@ struct DecodeMap {
     return {lo / 32, hi > lo ? (hi + 31) / 32 - lo / 32 : 0};
   }
   __device__ __forceinline__ Keys keys(int s) const {
-    if (held) return {__builtin_amdgcn_readlane(first, s), __builtin_amdgcn_readlane(n, s)};
+    if constexpr (HELD)
+      return {__builtin_amdgcn_readlane(first, s), __builtin_amdgcn_readlane(n, s)};
     if (p->cu_seqlens_q == nullptr) return range(p->seqlen_q, p->seqlen_k);
     return range(p->cu_seqlens_q[s + 1] - p->cu_seqlens_q[s],
                  p->cu_seqlens_k[s + 1] - p->cu_seqlens_k[s]);
   }
   __device__ __forceinline__ Seq seq(int s) const {
-    if (!held) return resolve_seq(*p, s);
+    if constexpr (!HELD) return resolve_seq(*p, s);
     Seq r;
     r.packed = true;
     r.lq = __builtin_amdgcn_readlane(lq, s);
@@ -1070,12 +1073,7 @@ struct DecodeMap {
   }
   __device__ __forceinline__ void init(const g4_problem& prob) {
     p = &prob;
-    held = p->cu_seqlens_q != nullptr && p->num_seqs <= 64;
-    if (p->cu_seqlens_q == nullptr) {
-      total = keys(0).n * p->num_seqs * p->num_kv_heads;
-      return;
-    }
-    if (held) {
+    if constexpr (HELD) {
       const int s = min((int)__lane_id(), p->num_seqs - 1);
       q0 = p->cu_seqlens_q[s];
       k0 = p->cu_seqlens_k[s];
@@ -1089,6 +1087,10 @@ struct DecodeMap {
       total = __builtin_amdgcn_readlane(end, 63) * p->num_kv_heads;
       return;
     }
+    if (p->cu_seqlens_q == nullptr) {
+      total = keys(0).n * p->num_seqs * p->num_kv_heads;
+      return;
+    }
     int sum = 0;
     for (int s = __lane_id(); s < p->num_seqs; s += 64) sum += keys(s).n;
     total = __builtin_amdgcn_readlane(scan(sum), 63) * p->num_kv_heads;
@@ -1096,15 +1098,15 @@ struct DecodeMap {
   // Sequence s that holds position pos < total, and its first position.
   __device__ __forceinline__ void find(int pos, int& s, int& first_pos) const {
     const int hkv = p->num_kv_heads;
+    if constexpr (HELD) {
+      s = __builtin_amdgcn_readfirstlane(__popcll(__ballot(start + n * hkv <= pos)));
+      first_pos = __builtin_amdgcn_readlane(start, s);
+      return;
+    }
     if (p->cu_seqlens_q == nullptr) {
       const int per = keys(0).n * hkv;
       s = pos / per;
       first_pos = s * per;
-      return;
-    }
-    if (held) {
-      s = __builtin_amdgcn_readfirstlane(__popcll(__ballot(start + n * hkv <= pos)));
-      first_pos = __builtin_amdgcn_readlane(start, s);
       return;
     }
     first_pos = 0;
@@ -1125,7 +1127,7 @@ struct DecodeMap {
   }
   // First position of sequence s.
   __device__ __forceinline__ int start_of(int s) const {
-    if (held) return __builtin_amdgcn_readlane(start, s);
+    if constexpr (HELD) return __builtin_amdgcn_readlane(start, s);
     if (p->cu_seqlens_q == nullptr) return s * keys(0).n * p->num_kv_heads;
     int sum = 0;
     for (int t = __lane_id(); t < s; t += 64) sum += keys(t).n;
@@ -1186,23 +1188,17 @@ struct DecodeKernel {
     __builtin_amdgcn_sched_barrier(0);
     row_steps<C::kNC, 4>(krd, smem + C::kLdsK, sv, qf);
     __builtin_amdgcn_sched_barrier(0);
-    if constexpr (C::kNW > 1) {
-      char G4_LDS* xb = smem + C::kLdsX;
+    char G4_LDS* xb = smem + C::kLdsX;
 #pragma unroll
-      for (int q4 = 0; q4 < 4; ++q4)
-        *(f32x4 G4_LDS*)(xb + ((dh * 4 + q4) * 64 + lane) * 16) =
-            f32x4{sv[q4 * 4], sv[q4 * 4 + 1], sv[q4 * 4 + 2], sv[q4 * 4 + 3]};
-      barrier_lds();
+    for (int q4 = 0; q4 < 4; ++q4)
+      *(f32x4 G4_LDS*)(xb + ((dh * 4 + q4) * 64 + lane) * 16) =
+          f32x4{sv[q4 * 4], sv[q4 * 4 + 1], sv[q4 * 4 + 2], sv[q4 * 4 + 3]};
+    barrier_lds();
 #pragma unroll
-      for (int q4 = 0; q4 < 4; ++q4) {
-        const f32x4 v = *(const f32x4 G4_LDS*)(xb + (((dh ^ 1) * 4 + q4) * 64 + lane) * 16);
-        // added in slice order, so that both slices hold the same scores
+    for (int q4 = 0; q4 < 4; ++q4) {
+      const f32x4 v = *(const f32x4 G4_LDS*)(xb + (((dh ^ 1) * 4 + q4) * 64 + lane) * 16);
 #pragma unroll
-        for (int e = 0; e < 4; ++e) {
-          const float mine = sv[q4 * 4 + e];
-          sv[q4 * 4 + e] = dh == 0 ? mine + v[e] : v[e] + mine;
-        }
-      }
+      for (int e = 0; e < 4; ++e) sv[q4 * 4 + e] += v[e];  // (the same sum in both slices)
     }
     if (more) issue_k(t + 1);  // every wave is done with K(t)
 
@@ -1252,7 +1248,7 @@ struct DecodeKernel {
   }
 };
 
-template <int D>
+template <int D, bool HELD>
 __global__ void __launch_bounds__(D / 4) fwd_decode_kernel(FwdParams a) {
   using K = DecodeKernel<D>;
   using C = typename K::C;
@@ -1273,7 +1269,7 @@ __global__ void __launch_bounds__(D / 4) fwd_decode_kernel(FwdParams a) {
   const int rows = grp * p.seqlen_q;  // row stride of the partial slots
 
   const int g = xcd_remap(blockIdx.x, gridDim.x);
-  DecodeMap map;
+  DecodeMap<HELD> map;
   map.init(p);
   const int n = min(a.split_chunks, map.total);  // (every part holds a tile)
   if (g >= n) return;
@@ -1282,7 +1278,7 @@ __global__ void __launch_bounds__(D / 4) fwd_decode_kernel(FwdParams a) {
   int s, start;
   map.find(pos, s, start);
   while (pos < end) {
-    const DecodeMap::Keys keys = map.keys(s);
+    const auto keys = map.keys(s);
     if (keys.n == 0) {
       ++s;
       continue;
@@ -1350,7 +1346,7 @@ __global__ void __launch_bounds__(D / 4) fwd_decode_kernel(FwdParams a) {
 // part, reading its maximum, sum and row one after the other; 6.2 us like this.
 // Q = 4 while the rows alone are fewer workgroups than CUs (16 sequences, 512
 // rows of about ten parts: Q = 4 12.8 us, Q = 1 9.0).
-template <int D, int Q>
+template <int D, int Q, bool HELD>
 __global__ void __launch_bounds__(256) merge_decode_kernel(FwdParams a) {
   constexpr int kCols = D / Q;          // columns of a workgroup
   constexpr int kLanes = kCols / 4;     // 16-byte loads of one part's row
@@ -1365,7 +1361,7 @@ __global__ void __launch_bounds__(256) merge_decode_kernel(FwdParams a) {
   const int quarter = blockIdx.x % Q;
   const int seg = blockIdx.x / Q / rows, r = blockIdx.x / Q % rows;
   const int s = seg / p.num_kv_heads, kvh = seg % p.num_kv_heads;
-  DecodeMap map;
+  DecodeMap<HELD> map;
   map.init(p);
   const Seq sq = map.seq(s);
   if (r >= grp * sq.lq) return;
@@ -1435,22 +1431,23 @@ __global__ void __launch_bounds__(256) merge_decode_kernel(FwdParams a) {
     a.lse[lse_off(p, sq, s, qh, qi)] = l > 0.f ? (mx + fast_log2(l)) * kLn2 : kNegInf;
 }
 
-template <int D>
+template <int D, bool HELD>
 static hipError_t launch_fwd_decode(const FwdParams& a, hipStream_t stream) {
   using C = DecodeCfg<D>;
   static LdsAttr attr;
-  hipError_t e = attr.ensure((const void*)fwd_decode_kernel<D>, C::kLdsBytes);
+  hipError_t e = attr.ensure((const void*)fwd_decode_kernel<D, HELD>, C::kLdsBytes);
   if (e != hipSuccess) return e;
   const int64_t rows = (int64_t)a.num_seqs * a.p.num_q_heads * a.p.seqlen_q;
-  hipLaunchKernelGGL(fwd_decode_kernel<D>, dim3((unsigned)a.split_chunks), dim3(C::kNW * 64),
-                     C::kLdsBytes, stream, a);
+  hipLaunchKernelGGL((fwd_decode_kernel<D, HELD>), dim3((unsigned)a.split_chunks),
+                     dim3(C::kNW * 64), C::kLdsBytes, stream, a);
   e = hipGetLastError();
   if (e != hipSuccess) return e;
   if (rows < 256)
-    hipLaunchKernelGGL((merge_decode_kernel<D, 4>), dim3((unsigned)(rows * 4)), dim3(256), 0,
+    hipLaunchKernelGGL((merge_decode_kernel<D, 4, HELD>), dim3((unsigned)(rows * 4)), dim3(256), 0,
                        stream, a);
   else
-    hipLaunchKernelGGL((merge_decode_kernel<D, 1>), dim3((unsigned)rows), dim3(256), 0, stream, a);
+    hipLaunchKernelGGL((merge_decode_kernel<D, 1, HELD>), dim3((unsigned)rows), dim3(256), 0,
+                       stream, a);
   return hipGetLastError();
 }
 
@@ -2153,7 +2150,9 @@ __global__ void clear_list_kernel(unsigned* n) {
 }
 
 hipError_t launch_fwd(const FwdParams& a, hipStream_t stream) {
-  if (a.split_slots > 0) return launch_fwd_decode<512>(a, stream);
+  if (a.split_slots > 0)
+    return a.p.cu_seqlens_q != nullptr && a.num_seqs <= 64 ? launch_fwd_decode<512, true>(a, stream)
+                                                           : launch_fwd_decode<512, false>(a, stream);
   if (a.split_chunks > 0) {
     if (a.p.head_dim == 256) return launch_fwd_split<256>(a, stream);
     if (a.p.head_dim == 512) return launch_fwd_split<512>(a, stream);
