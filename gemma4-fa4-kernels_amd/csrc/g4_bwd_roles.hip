@@ -137,9 +137,11 @@ struct SplitRun {
 // LDS (this wave's own, 16-byte chunks swizzled by row) and leaves as 256-byte
 // row segments: dK/dV of 131072 local tokens 12.55 -> 12.43 ms, of 32 global
 // sequences (32768 tokens) 3.61 -> 3.57, of 8192 local tokens 0.870 -> 0.857.
-// (The split launch at head dim 512 keeps the direct stores for its few whole
-// tiles: with these its step loop took other registers, 115 -> 126 us at 1000
-// tokens.)  row(r) is the address of key r's first column; keys from nrows on
+// (At head dim 512 only the work queue's launch takes it.  One workgroup per item
+// waits for the stage at the end of its few items: 600 tokens 358 us direct, 364
+// staged, 8 x 300 229 / 235, with GQA 1 87 / 105.  In the split launch, for its few
+// whole tiles, the step loop took other registers: 115 -> 126 us at 1000 tokens.)
+// row(r) is the address of key r's first column; keys from nrows on
 // are not stored.
 template <class Row>
 __device__ __forceinline__ void store_key_rows(const f32x16 (&acc)[8], char G4_LDS* stage,
@@ -455,7 +457,7 @@ struct RolesKernel {
 
     if constexpr (SPLIT)
       if (part != nullptr) return store_split_part(part, acc, wave, lane);
-    if constexpr (!STRIPED && !SPLIT) {
+    if constexpr (!STRIPED && !SPLIT && !ROT) {
       barrier_lds();  // every wave is done with the tiles
       const int jw = j0 + kb * 32;  // this wave's first key
       const g4_layout& ly = PWAVE ? a->dvl : a->dkl;
