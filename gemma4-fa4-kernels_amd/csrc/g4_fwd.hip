@@ -1596,8 +1596,9 @@ __device__ __forceinline__ int wide_tile(int r, int n) {
 }
 
 // Tiles of a run of WideItem::decode_equal (1: 8192 tokens 1% slower, 3 x 2000
-// tokens alike; 8: 3 x 2000 tokens 1% slower).
+// tokens alike; 8: 3 x 2000 tokens 1% slower), and of a batch on one XCD.
 constexpr int kEqualRun = 4;
+constexpr int kEqualBatch = 64;
 
 // Query tile of a wide workgroup: KV head kvh, key chunk, sequence s, tile qt.
 struct WideItem {
@@ -1627,19 +1628,46 @@ struct WideItem {
   // Item of workgroup b of a launch without a split over sequences of equal
   // length.  The (sequence, KV head) segments fall into as many equal sets as
   // XCDs allow (the largest power of two up to 8 that divides them), each set
-  // on an equal number of XCDs, whose workgroups take its segments one after the
-  // other, each from its last tile to its first, kEqualRun adjacent tiles at a
-  // time: heavy tiles begin first, light ones fill the end, and an XCD's
-  // neighbours cost alike and share K and V.
+  // on an equal number of XCDs, which take kEqualRun adjacent tiles at a time, the
+  // last tiles first: heavy ones begin first, light ones fill the end, and an XCD's
+  // neighbours cost alike and share K and V.  A set of several segments takes them
+  // in batches of about two rounds of its CUs, the runs of a batch's segments in
+  // turn, so that no segment's heavy tiles begin when the others' light ones end (one
+  // segment after the other 8 heads of 4 x 2048 tokens, GQA 1, took 234 us, in zigzag
+  // ranks 212, so 180; all segments in one batch lose the shared K and V: 32 heads of
+  // 5 x 1300 517 us, 468 in batches).  Within a run the tiles rotate from run to run: the
+  // hardware deals neighbours to the four shader engines of an XCD in turn, and each
+  // would get the same tile of every segment.  Up to kEqualRun tiles in all, the
+  // segments' last tiles come first, then the ones before (16 x 500, 8 heads 93 / 76).
   __device__ __forceinline__ bool decode_equal(const FwdParams& a, int b) {
     constexpr int kXcd = 8;
     const int segs = a.num_seqs * a.p.num_kv_heads;
     const int sets = min(segs & -segs, kXcd), per_set = segs / sets, xcds = kXcd / sets;
-    const int x = b % kXcd, p = b / kXcd, sub = x & (xcds - 1), run = p / kEqualRun;
-    const int r = (run * xcds + (run & 1 ? xcds - 1 - sub : sub)) * kEqualRun + p % kEqualRun;
+    const int x = b % kXcd, p = b / kXcd, sub = x & (xcds - 1), turn = p / kEqualRun;
+    int r = (turn * xcds + (turn & 1 ? xcds - 1 - sub : sub)) * kEqualRun + p % kEqualRun;
     if (r >= per_set * a.ntq) return false;
-    const int seg = x / xcds * per_set + r / a.ntq;
-    qt = a.ntq - 1 - r % a.ntq;
+    int seg = x / xcds * per_set;
+    if (per_set > 1) {
+      const int batches = max(per_set * a.ntq / (kEqualBatch * xcds), 1);
+      const int batch = (per_set + batches - 1) / batches;
+      seg += r / (batch * a.ntq) * batch;
+      r %= batch * a.ntq;
+      const int n = min(batch, (x / xcds + 1) * per_set - seg);  // segments of this batch
+      const int full = a.ntq / kEqualRun * kEqualRun * n, rem = a.ntq % kEqualRun;
+      if (a.ntq <= kEqualRun) {
+        seg += r % n;
+        r /= n;
+      } else if (r < full) {
+        const int run = r / kEqualRun;
+        seg += run % n;
+        r = run / n * kEqualRun + (r + run) % kEqualRun;
+      } else {
+        r -= full;
+        seg += r / rem;
+        r = a.ntq - rem + (r + (rem == 2 ? r / rem / 2 : 0)) % rem;
+      }
+    }
+    qt = a.ntq - 1 - r;
     s = seg / a.p.num_kv_heads;
     kvh = seg - s * a.p.num_kv_heads;
     chunk = row_tile = 0;

@@ -29,6 +29,11 @@ CASES = [
     (16, 16, 1, 385, False),
     (24, 12, 2, 130, False),
     (32, 4, 4, 70, False),
+    # several segments in a set: up to four tiles each, remainders of 2 and 3, two batches
+    (6, 6, 8, 300, False),
+    (16, 16, 3, 650, False),
+    (3, 3, 6, 1300, False),
+    (16, 16, 8, 900, False),
 ]
 
 
